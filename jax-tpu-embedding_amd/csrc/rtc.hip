@@ -162,7 +162,7 @@ struct Entry {
 // Compiles program p for one layout on the current device (architecture
 // arch) and loads the result.
 Entry Compile(const DevProgram& p, const std::string& arch, int g, int vec,
-              int src, int unroll, bool mapped) {
+              int src, bool one_hot, bool mapped) {
   Entry e;
   const Hiprtc& rtc = GetHiprtc();
   if (rtc.create == nullptr) {
@@ -184,7 +184,8 @@ Entry Compile(const DevProgram& p, const std::string& arch, int g, int vec,
   const std::string m = mapped ? "true" : "false";
   const std::string reduce_expr =
       "&scemb::SegReduce<" + layout + ", " + std::to_string(src) + ", " +
-      std::to_string(kEpiRtc) + ", " + std::to_string(unroll) + ", " + m + ">";
+      std::to_string(kEpiRtc) + ", " + (one_hot ? "true" : "false") + ", " + m +
+      ", " + std::to_string(g) + ">";
   const std::string finish_expr = "&scemb::SegFinish<" + layout + ", " +
                                   std::to_string(kEpiRtc) + ", " + m + ">";
   hiprtcProgram prog;
@@ -250,7 +251,7 @@ Entry Compile(const DevProgram& p, const std::string& arch, int g, int vec,
 
 }  // namespace
 
-int RtcKernelsFor(const DevProgram& p, int g, int vec, int src, int unroll,
+int RtcKernelsFor(const DevProgram& p, int g, int vec, int src, bool one_hot,
                   bool mapped, RtcKernels* k) {
   const Mode mode = GetMode();
   if (mode == Mode::kUnknown) {
@@ -264,7 +265,7 @@ int RtcKernelsFor(const DevProgram& p, int g, int vec, int src, int unroll,
   // and the transcendental flag follow from them).
   char head[96];
   std::snprintf(head, sizeof(head), "%d:%d:%d:%d:%d:%d:%d:%d:%d:%u:", dev, g,
-                vec, src, unroll, mapped ? 1 : 0, p.num_ops, p.num_slots,
+                vec, src, one_hot ? 1 : 0, mapped ? 1 : 0, p.num_ops, p.num_slots,
                 p.num_hyper, p.out);
   std::string key(head);
   key.append(reinterpret_cast<const char*>(p.code),
@@ -278,7 +279,7 @@ int RtcKernelsFor(const DevProgram& p, int g, int vec, int src, int unroll,
   if (it == cache->end()) {
     hipDeviceProp_t prop;
     SCEMB_HIP(hipGetDeviceProperties(&prop, dev));
-    it = cache->emplace(key, Compile(p, prop.gcnArchName, g, vec, src, unroll,
+    it = cache->emplace(key, Compile(p, prop.gcnArchName, g, vec, src, one_hot,
                                      mapped)).first;
   }
   const Entry e = it->second;

@@ -17,11 +17,11 @@
 //   * a sample view built once per preprocessed batch (forward);
 //   * otherwise ExpandCsr + a stable radix sort inside the call.
 //
-// SegReduce gives every 256-thread block a fixed slice of 256 stream entries
-// (perfect load balance however skewed the keys are). A block is split into
-// P = 256 / G sub-groups of G lanes; sub-group s owns entries [s*G, s*G + G)
+// SegReduce gives every 256-thread block a fixed slice of the stream (perfect
+// load balance however skewed the keys are). A block is split into
+// P = 256 / G sub-groups of G lanes; sub-group s owns entries [s*R, s*R + R)
 // of the slice and its lanes cover G * VEC columns of a row (16-byte loads).
-// A sub-group walks its entries kUnroll at a time, issuing all row loads of a
+// A sub-group walks its entries a few at a time, issuing all row loads of a
 // batch (and, for runs that end inside the batch, the table / accumulator
 // loads of the update) before accumulating. A run that is complete inside
 // one sub-group is finished there; pieces of runs that cross sub-groups are
@@ -181,30 +181,51 @@ struct RtcKernels {
   hipFunction_t finish;
 };
 
-// The kernels of program p for layout (g, vec, src, unroll, mapped) on the
+// The kernels of program p for layout (g, vec, src, one_hot, mapped) on the
 // current device, compiled at the first request and kept for the process.
 // 0: *k is set. kRtcInterpret: interpret the program instead (compilation
 // switched off, or unavailable or failed while not required). Otherwise an
 // error code (SCEMB_ERR_*), message set: SCEMB_CUSTOM_UPDATE unknown, or
 // compilation required (SCEMB_CUSTOM_UPDATE=compile) and failed.
 constexpr int kRtcInterpret = -1;
-int RtcKernelsFor(const DevProgram& p, int g, int vec, int src, int unroll,
+int RtcKernelsFor(const DevProgram& p, int g, int vec, int src, bool one_hot,
                   bool mapped, RtcKernels* k);
 #endif  // __HIPCC_RTC__
 
 namespace {
 
 
-constexpr int kBlock = 256;  // threads per block = stream entries per block
+constexpr int kBlock = 256;  // threads per block; entries per hot-run mark
+
+// Whether rows are summed with fused multiply-adds, in ranges of any length:
+// the lookup. The updates keep the order of one multiply and one add per
+// entry in ranges of G, which every update shares (a custom program's result
+// equals the built-in optimizer's bit for bit). It also keeps the last bits of
+// hot rows where they count: such a row adds up 1e5 gradients that nearly
+// cancel, and where that leaves a sum near zero, Adagrad's square root turned
+// another order of it into 1e-6 of the size of a later lookup's columns. Of
+// the update of two weighted multi-hot stacks (4.3M entries, 64 columns, SGD)
+// it costs 449 us against 412.
+template <int EPI>
+__host__ __device__ constexpr bool AnyOrder() {
+  return EPI == kEpiFwd;
+}
+
 // Entries whose rows a sub-group loads together (memory-level parallelism;
 // the backward also holds the table / accumulator rows of the runs that end
 // in the batch). Batches of about one entry per activation row ("one-hot")
 // gain from the wide setting; multi-hot batches, whose gathers mostly hit
-// cache, from the higher occupancy of the narrow one (fewer registers).
-constexpr int kFwdUnrollWide = 8;
-constexpr int kFwdUnrollNarrow = 4;
-constexpr int kBwdUnrollWide = 4;
-constexpr int kBwdUnrollNarrow = 2;
+// cache, from the higher occupancy of the narrow one (fewer registers): 8
+// instead of 4 entries slowed a weighted multi-hot lookup (two stacks of
+// 4.3M entries, 64 columns) from 198 to 222 us. SGD holds no slot rows and
+// takes 4 there too (update of the same stacks, summed with fused
+// multiply-adds: 441 us with 2, 413 with 4);
+// with slots 4 gained nothing (Adagrad, 128 columns: 905 and 911 us).
+template <int EPI, bool kOneHot>
+__host__ __device__ constexpr int Unroll() {
+  return EPI == kEpiFwd ? (kOneHot ? 8 : 4)
+                        : (kOneHot || EPI == kEpiSgd ? 4 : 2);
+}
 // Entries per activation row up to which a batch counts as one-hot.
 constexpr int64_t kOneHotMaxEntriesPerRow = 2;
 // Streaming (nontemporal) access for data touched once per call, so the
@@ -498,7 +519,6 @@ struct RowArgs {
   float* slot1;
   int64_t dim;
   int64_t batch;     // forward: rows of dst
-  bool stream_src;   // gathered rows are read about once: nontemporal loads
   RowMap act;        // activation layout (dst forward, src backward)
   OptParams opt;
   float* partials;   // [2 * num_blocks, dim]
@@ -1104,20 +1124,94 @@ __device__ __forceinline__ void ZeroRows(const RowMapLds& m, float* dst,
   }
 }
 
-template <int G, int VEC, int SRC, int EPI, int kUnroll, bool kMapped>
+// What a sub-group does after entry i of its range: nothing (the run goes
+// on), finish the run here, leave a piece for the block's combine (a run from
+// the range before, or one that continues past the range), or drop the sum
+// (padding and invalid entries, each a run of its own).
+enum { kActNone = 0, kActFinish = 1, kActHead = 2, kActTail = 3, kActDrop = 4 };
+constexpr uint32_t kActMask = 7;
+constexpr int kActBits = 3;
+// Columns that a mapped entry's gathered row has, in the bits above the
+// action; all ones: every column.
+constexpr uint32_t kAllColumns = 0xffffffffu >> kActBits;
+
+// One stream entry as the reduction reads it, 16 bytes in LDS: the address of
+// its gathered row, its gain, and action | columns << kActBits.
+struct __attribute__((aligned(16))) SegEntry {
+  const float* row;
+  float gain;
+  uint32_t info;
+};
+
+// Address of activation row `row` in a row map and the columns it has there
+// (null and 0: in no block).
+__device__ __forceinline__ float* ActRow(const RowMapLds& m, int64_t dim,
+                                         int64_t row, uint32_t* columns) {
+  *columns = 0;
+  if (m.n == 0) return nullptr;
+  int lo = 0, hi = m.n;  // last block whose first row is <= row
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (m.first[mid] <= row) lo = mid; else hi = mid;
+  }
+  if (row < m.first[lo] || row >= m.end[lo]) return nullptr;
+  const int32_t w = m.width[lo];
+  *columns = w >= dim ? kAllColumns
+             : static_cast<uint32_t>(w) < kAllColumns
+                 ? static_cast<uint32_t>(w)
+                 : kAllColumns - 1;
+  return m.data[lo] + (row - m.first[lo]) * m.stride[lo];
+}
+
+// Key of stream entry e, or kSkip where it belongs to a hot run.
+template <int SRC>
+__device__ __forceinline__ uint32_t FetchCold(const StreamArgs& s, bool hot,
+                                              int64_t e, uint64_t* ent,
+                                              uint32_t* status) {
+  if (hot) {
+    int lead, trail;
+    HotSpan(s, e / kBlock, &lead, &trail);
+    const int i = static_cast<int>(e % kBlock);
+    if (i < lead || i >= trail) {
+      *ent = 0;
+      return kSkip;
+    }
+  }
+  return FetchEntry<SRC>(s, e, ent, status);
+}
+
+// One block reduces kBlock / G sub-groups' ranges of R consecutive entries.
+// What bounds it with several entries per run is instruction issue, not
+// memory: with the entry's masks, its action and its row's address worked out
+// by every lane at every step, a step took about 45 vector and 43 scalar
+// instructions to load 16 bytes a lane and add them. So the thread that
+// stages an entry works them out once, and a step is one 16-byte LDS read,
+// one 64-bit add, the load and four fused multiply-adds.
+template <int G, int VEC, int SRC, int EPI, bool kOneHot, bool kMapped, int R>
 __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
   using V = Vec<VEC>;
   using T = typename V::T;
   constexpr int P = kBlock / G;
-  __shared__ uint32_t s_key[kBlock + 2];  // [0]: entry before, [257]: after
-  __shared__ uint64_t s_ent[kBlock];
+  constexpr int kSpan = P * R;                 // entries per block
+  constexpr int kWaveSpan = kWave / G * R;     // entries per wave
+  constexpr int kChunks = kWaveSpan / kWave;   // entries per thread, staged
+  constexpr int kUnroll = Unroll<EPI, kOneHot>();
+  constexpr int U = kUnroll < R ? kUnroll : R;
+  static_assert(R >= G && R <= kWave && kWave % R == 0 && R % U == 0, "range");
+  // Gathered rows read about once (one-hot batches): nontemporal loads.
+  constexpr bool kStreamSrc = EPI != kEpiFwd && kOneHot;
+  __shared__ uint32_t s_key[kSpan + 2];  // [0]: entry before, last: after
+  __shared__ SegEntry s_ent[kSpan];
   __shared__ T s_part[2 * P][G];
   __shared__ uint32_t s_info[P];
+  __shared__ uint32_t s_range[P];  // first entry, end of the last, in a range
+  __shared__ float* s_dst[EPI == kEpiFwd && kMapped ? kSpan : 1];
+  __shared__ uint32_t s_dcols[EPI == kEpiFwd && kMapped ? kSpan : 1];
   __shared__ RowMapLds s_map;
 
   const int tid = threadIdx.x;
   const int64_t blk = blockIdx.x;
-  const int64_t cb = blk * kBlock;
+  const int64_t cb = blk * kSpan;
   const int64_t n = st.n;
   // Blocks that lie wholly in the padding after the last entry (CSR buffers
   // are sized for the worst case) only clear their flag: with the CSR, past
@@ -1146,115 +1240,161 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
   // Entries of hot runs read as outside any run; a block of nothing else
   // has no work.
   const bool hot = SRC == kSrcCsr && st.hot_head != nullptr;
-  int lead = 0, trail = kBlock;
   if (hot) {
-    HotSpan(st, blk, &lead, &trail);
-    if (lead >= trail) {
+    bool cold = false;
+    for (int64_t b = cb / kBlock; b < (cb + kSpan) / kBlock && b * kBlock < n;
+         ++b) {
+      int lead, trail;
+      HotSpan(st, b, &lead, &trail);
+      cold = cold || lead < trail;
+    }
+    if (!cold) {
       if (tid == 0) r.block_flags[blk] = 0;
       return;
     }
   }
-  if (kMapped) StageRowMap(r.act, &s_map);
-  {
+  if (kMapped) {
+    StageRowMap(r.act, &s_map);
+    __syncthreads();
+  }
+  const int64_t dim = r.dim;
+  const int wave = tid / kWave;
+  const int lane = tid % kWave;
+  uint32_t key[kChunks];
+  uint32_t columns[kChunks];
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const int i = wave * kWaveSpan + c * kWave + lane;
     uint64_t en = 0;
-    uint32_t k = kSkip;
-    if (cb + tid < n && tid >= lead && tid < trail) {
-      k = FetchEntry<SRC>(st, cb + tid, &en, r.status);
-    }
-    s_key[tid + 1] = k;
-    s_ent[tid] = en;
-    if (tid == 0) {
-      uint64_t d;
-      bool skip = cb == 0;
-      if (!skip && hot) {
-        int l, t;
-        HotSpan(st, blk - 1, &l, &t);
-        skip = kBlock - 1 < l || kBlock - 1 >= t;
+    key[c] = cb + i < n ? FetchCold<SRC>(st, hot, cb + i, &en, r.status)
+                        : kSkip;
+    s_key[i + 1] = key[c];
+    columns[c] = kAllColumns;
+    // Entries outside any run read a row that is there and drop it.
+    const float* row = r.src;
+    if (EPI != kEpiFwd && kMapped) {
+      columns[c] = 0;
+      if (key[c] != kSkip) {
+        row = ActRow(s_map, dim, PackedIndex(en), &columns[c]);
       }
-      s_key[0] = skip ? kSkip : FetchEntry<SRC>(st, cb - 1, &d, nullptr);
+    } else if (key[c] != kSkip) {
+      row = r.src + static_cast<int64_t>(PackedIndex(en)) * dim;
     }
-    if (tid == kBlock - 1) {
-      uint64_t d;
-      bool skip = cb + kBlock >= n;
-      if (!skip && hot) {
-        int l, t;
-        HotSpan(st, blk + 1, &l, &t);
-        skip = 0 < l || 0 >= t;
+    if (EPI == kEpiFwd && kMapped) {
+      s_dst[i] = nullptr;
+      s_dcols[i] = 0;
+      if (key[c] != kSkip) {
+        s_dst[i] = ActRow(s_map, dim, key[c], &s_dcols[i]);
       }
-      s_key[kBlock + 1] =
-          skip ? kSkip : FetchEntry<SRC>(st, cb + kBlock, &d, nullptr);
     }
+    s_ent[i].row = row;
+    s_ent[i].gain = PackedGain(en);
+  }
+  if (tid == 0) {
+    uint64_t d;
+    s_key[0] = cb == 0 ? kSkip : FetchCold<SRC>(st, hot, cb - 1, &d, nullptr);
+  }
+  if (tid == kBlock - 1) {
+    uint64_t d;
+    s_key[kSpan + 1] = cb + kSpan >= n
+                           ? kSkip
+                           : FetchCold<SRC>(st, hot, cb + kSpan, &d, nullptr);
   }
   __syncthreads();
 
-  const int sub = tid / G;
-  const int cl = tid % G;
-  const int base = sub * G;  // first entry of the sub-group in the block
-  const int64_t left = n - (cb + base);
-  const int cnt = left <= 0 ? 0 : (left < G ? static_cast<int>(left) : G);
-  const uint32_t my_key = s_key[tid + 1];
-  const uint32_t prev_key = s_key[tid];
-  const bool mine = cl < cnt;
-  const bool valid = mine && my_key != kSkip;
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const int i = wave * kWaveSpan + c * kWave + lane;
+    const int64_t e = cb + i;
+    const uint32_t my_key = key[c];
+    const uint32_t prev_key = s_key[i];
+    const uint32_t next_key = s_key[i + 2];
+    const bool mine = e < n;
+    const bool valid = my_key != kSkip;
 
-  // A minibatched CSR is contiguous by row but not ascending (a minibatch's
-  // buckets follow each other); that cannot be checked locally.
-  if (r.status != nullptr && mine &&
-      (SRC != kSrcCsr || st.csr.num_minibatches == 0)) {
-    const bool bad = SRC == kSrcCsr
-                         ? (valid && prev_key != kSkip && prev_key > my_key)
-                         : (cb + tid > 0 && prev_key > my_key);
-    if (bad) atomicOr(r.status, SCEMB_STATUS_UNSORTED);
-  }
-
-  const int wshift = (tid % kWave) / G * G;
-  const uint64_t gmask = LowBits(G);
-  const uint64_t valid_m = (__ballot(valid) >> wshift) & gmask;
-  const uint64_t start_m =
-      (__ballot(valid && my_key != prev_key) >> wshift) & gmask;
-  const uint64_t end_m =
-      (__ballot(valid && (cl == cnt - 1 || my_key != s_key[tid + 2])) >>
-       wshift) & gmask;
-
-  if (EPI == kEpiFwd) {
-    // Activation rows without entries: rows strictly between the clamped
-    // keys of consecutive entries, before the first and after the last.
-    const int64_t e = cb + tid;
-    const int64_t ck = my_key == kSkip ? r.batch : my_key;
-    const int64_t cp = e == 0 ? -1 : (prev_key == kSkip ? r.batch : prev_key);
-    const bool gap = mine && ck > cp + 1;
-    uint64_t m = (__ballot(gap) >> wshift) & gmask;
-    while (m) {
-      const int l = __ffsll(static_cast<long long>(m)) - 1;
-      m &= m - 1;
-      const int64_t lo = __shfl(static_cast<int>(cp + 1), wshift + l);
-      const int64_t hi = __shfl(static_cast<int>(ck), wshift + l);
-      ZeroRows<G, VEC, kMapped>(s_map, r.dst, r.dim, lo, hi, cl);
+    // A minibatched CSR is contiguous by row but not ascending (a
+    // minibatch's buckets follow each other); that cannot be checked
+    // locally.
+    if (r.status != nullptr && mine &&
+        (SRC != kSrcCsr || st.csr.num_minibatches == 0)) {
+      const bool bad = SRC == kSrcCsr
+                           ? (valid && prev_key != kSkip && prev_key > my_key)
+                           : (e > 0 && prev_key > my_key);
+      if (bad) atomicOr(r.status, SCEMB_STATUS_UNSORTED);
     }
-    const bool tail_gap = mine && e == n - 1 && ck + 1 < r.batch;
-    m = (__ballot(tail_gap) >> wshift) & gmask;
-    if (m) {
-      const int l = __ffsll(static_cast<long long>(m)) - 1;
-      const int64_t lo = __shfl(static_cast<int>(ck + 1), wshift + l);
-      ZeroRows<G, VEC, kMapped>(s_map, r.dst, r.dim, lo, r.batch, cl);
+
+    if (EPI == kEpiFwd) {
+      // Activation rows without entries: rows strictly between the clamped
+      // keys of consecutive entries, before the first and after the last.
+      // The lanes of a sub-group's width clear those of their entries.
+      const int cl = lane % G;
+      const int wshift = lane / G * G;
+      const uint64_t gmask = LowBits(G);
+      const int64_t ck = my_key == kSkip ? r.batch : my_key;
+      const int64_t cp =
+          e == 0 ? -1 : (prev_key == kSkip ? r.batch : prev_key);
+      const bool gap = mine && ck > cp + 1;
+      uint64_t m = (__ballot(gap) >> wshift) & gmask;
+      while (m) {
+        const int l = __ffsll(static_cast<long long>(m)) - 1;
+        m &= m - 1;
+        const int64_t lo = __shfl(static_cast<int>(cp + 1), wshift + l);
+        const int64_t hi = __shfl(static_cast<int>(ck), wshift + l);
+        ZeroRows<G, VEC, kMapped>(s_map, r.dst, r.dim, lo, hi, cl);
+      }
+      const bool tail_gap = mine && e == n - 1 && ck + 1 < r.batch;
+      m = (__ballot(tail_gap) >> wshift) & gmask;
+      if (m) {
+        const int l = __ffsll(static_cast<long long>(m)) - 1;
+        const int64_t lo = __shfl(static_cast<int>(ck + 1), wshift + l);
+        ZeroRows<G, VEC, kMapped>(s_map, r.dst, r.dim, lo, r.batch, cl);
+      }
+    }
+
+    // What the entry's range does with it. A chunk of a wave's entries holds
+    // whole ranges.
+    const int j = lane % R;
+    const int rshift = lane / R * R;
+    const uint64_t rmask = LowBits(R);
+    const int64_t left = n - (e - j);
+    const int cnt = left <= 0 ? 0 : (left < R ? static_cast<int>(left) : R);
+    const uint64_t valid_m = (__ballot(valid) >> rshift) & rmask;
+    const uint64_t start_m =
+        (__ballot(valid && my_key != prev_key) >> rshift) & rmask;
+    const bool last = j == cnt - 1;
+    const bool goes_on = valid && my_key == next_key;
+    const bool tail_cont =
+        ((__ballot(last && goes_on) >> rshift) & rmask) != 0;
+    // Pieces of the range that are not whole runs.
+    const bool head_cont = (valid_m & 1) && !(start_m & 1);
+    const bool first = (start_m & ~1ull & LowBits(j + 1)) == 0;
+    const bool head_piece = head_cont && first;
+    uint32_t act = kActDrop;
+    if (valid) {
+      act = !(last || !goes_on)       ? kActNone
+            : head_piece              ? kActHead
+            : last && tail_cont       ? kActTail
+                                      : kActFinish;
+    }
+    s_ent[i].info = act | (columns[c] << kActBits);
+    if (j == 0) {
+      const bool whole = head_cont && tail_cont &&
+                         (start_m & ~1ull & LowBits(cnt)) == 0;
+      s_info[i / R] = (head_cont ? kHasHead : 0) |
+                      (head_cont && !whole ? kHeadEnds : 0) |
+                      (tail_cont && !whole ? kHasTail : 0);
+      s_range[i / R] =
+          valid_m == 0
+              ? 0u
+              : (static_cast<uint32_t>(
+                     __ffsll(static_cast<long long>(valid_m)) - 1) |
+                 (static_cast<uint32_t>(kWave - __clzll(static_cast<long long>(
+                                                    valid_m))) << 16));
     }
   }
 
-  // Pieces of this sub-group's range that are not whole runs.
-  const bool head_cont = (valid_m & 1) && !(start_m & 1);
-  bool tail_cont = false;
-  if (cnt > 0) {
-    const uint32_t kl = s_key[base + cnt];
-    tail_cont = kl != kSkip && kl == s_key[base + cnt + 1];
-  }
-  const bool whole = head_cont && tail_cont &&
-                     (start_m & ~1ull & LowBits(cnt)) == 0;
-  const uint32_t info = (head_cont ? kHasHead : 0) |
-                        (head_cont && !whole ? kHeadEnds : 0) |
-                        (tail_cont && !whole ? kHasTail : 0);
-  if (cl == 0) s_info[sub] = info;
   if (tid == 0) {
-    const int last = n - cb < kBlock ? static_cast<int>(n - cb) : kBlock;
+    const int last = n - cb < kSpan ? static_cast<int>(n - cb) : kSpan;
     const uint32_t kf = s_key[1], kl = s_key[last];
     const bool from_prev = kf != kSkip && kf == s_key[0];
     const bool to_next = kl != kSkip && kl == s_key[last + 1];
@@ -1270,79 +1410,80 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
       atomicOr(r.status, SCEMB_STATUS_SHARED_ROW);
     }
   }
+  __syncthreads();
 
+  const int sub = tid / G;
+  const int cl = tid % G;
+  const int base = sub * R;  // first entry of the sub-group in the block
+  const uint32_t info = s_info[sub];
+  const int range_lo = static_cast<int>(s_range[sub] & 0xffffu) / U * U;
+  const int range_hi = static_cast<int>(s_range[sub] >> 16);
   const Hyper H = LoadHyper<EPI>(r.opt);
-  const int64_t dim = r.dim;
   for (int64_t col0 = 0; col0 < dim; col0 += static_cast<int64_t>(G) * VEC) {
     const int64_t col = col0 + static_cast<int64_t>(cl) * VEC;
     const bool col_ok = col < dim;
+    // Lanes past the last column read along with the first.
+    const int64_t lcol = col_ok ? col : 0;
     T acc = V::Zero();
-    for (int q = 0; q < cnt; q += kUnroll) {
-      T v[kUnroll];
-      T tv[kUnroll];
-      T av[kUnroll];
-      T bv[kUnroll];
-      T res[kUnroll];  // interpreted updates: finished rows' gradient sums
-      float gn[kUnroll];
-      uint32_t kk[kUnroll];
-      bool fin[kUnroll];
+    for (int q = range_lo; q < range_hi; q += U) {
+      T v[U];
+      T tv[U];
+      T av[U];
+      T bv[U];
+      T res[U];  // interpreted updates: finished rows' gradient sums
+      float gn[U];
+      uint32_t act[U];
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int idx = q + u;
-        const bool val = idx < cnt && ((valid_m >> idx) & 1);
-        uint64_t en = 0;
-        kk[u] = kSkip;
-        if (val) {
-          en = s_ent[base + idx];
-          kk[u] = s_key[base + idx + 1];
+      for (int u = 0; u < U; ++u) {
+        const SegEntry en = s_ent[base + q + u];
+        act[u] = en.info & kActMask;
+        gn[u] = en.gain;
+        if (EPI != kEpiFwd && kMapped) {
+          const uint32_t w = en.info >> kActBits;
+          v[u] = V::Zero();
+          if (col_ok && (w == kAllColumns || lcol < w)) {
+            v[u] = LoadRow<VEC, kStreamSrc>(en.row + lcol);
+          }
+        } else {
+          v[u] = LoadRow<VEC, kStreamSrc>(en.row + lcol);
         }
-        gn[u] = PackedGain(en);
-        v[u] = V::Zero();
-        if (val && col_ok) {
-          // Forward: table rows (dense); backward: activation-gradient rows
-          // through the row map.
-          const float* p =
-              EPI == kEpiFwd
-                  ? r.src + static_cast<int64_t>(PackedIndex(en)) * dim + col
-                  : ActAddr<kMapped>(s_map, const_cast<float*>(r.src), dim,
-                                     PackedIndex(en), col);
-          if (p != nullptr) v[u] = r.stream_src ? V::LoadNT(p) : V::Load(p);
-        }
-        const bool is_end = val && ((end_m >> idx) & 1);
-        const bool first = (start_m & ~1ull & LowBits(idx + 1)) == 0;
-        const bool head_piece = head_cont && first;
-        const bool tail_piece = idx == cnt - 1 && tail_cont;
-        fin[u] = is_end && !head_piece && !tail_piece;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
         tv[u] = V::Zero();
         av[u] = V::Zero();
         bv[u] = V::Zero();
         res[u] = V::Zero();
-        if (EPI != kEpiFwd && fin[u] && col_ok) {
-          const int64_t off = static_cast<int64_t>(kk[u]) * dim + col;
+        if (EPI != kEpiFwd && act[u] == kActFinish && col_ok) {
+          const int64_t off =
+              static_cast<int64_t>(s_key[base + q + u + 1]) * dim + col;
           tv[u] = V::Load(r.dst + off);
           if (HasSlot<EPI>(r.opt, 0)) av[u] = V::Load(r.slot0 + off);
           if (HasSlot<EPI>(r.opt, 1)) bv[u] = V::Load(r.slot1 + off);
         }
       }
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int idx = q + u;
-        if (idx < cnt && ((valid_m >> idx) & 1)) {
-          acc = V::Fma(acc, gn[u], v[u]);
-          if ((end_m >> idx) & 1) {
-            if (fin[u]) {
-              if constexpr (IsInterpreted<EPI>()) {
-                res[u] = acc;  // updated below
-              } else if (col_ok) {
-                Epilogue<VEC, EPI, kMapped>(r, s_map, kk[u], col, acc, tv[u],
-                                            av[u], bv[u], H);
+      for (int u = 0; u < U; ++u) {
+        acc = AnyOrder<EPI>() ? V::Fused(acc, gn[u], v[u])
+                              : V::Fma(acc, gn[u], v[u]);
+        if (act[u] != kActNone) {
+          if (act[u] == kActFinish) {
+            if constexpr (IsInterpreted<EPI>()) {
+              res[u] = acc;  // updated below
+            } else if constexpr (EPI == kEpiFwd && kMapped) {
+              float* p = s_dst[base + q + u];
+              const uint32_t w = s_dcols[base + q + u];
+              if (p != nullptr && col_ok && (w == kAllColumns || col < w)) {
+                StoreRow<VEC, kNtAct>(p + col, acc);
               }
-            } else {
-              const bool first = (start_m & ~1ull & LowBits(idx + 1)) == 0;
-              s_part[head_cont && first ? 2 * sub : 2 * sub + 1][cl] = acc;
+            } else if (col_ok) {
+              Epilogue<VEC, EPI, kMapped>(r, s_map, s_key[base + q + u + 1],
+                                          col, acc, tv[u], av[u], bv[u], H);
             }
-            acc = V::Zero();
+          } else if (act[u] != kActDrop) {
+            s_part[act[u] == kActHead ? 2 * sub : 2 * sub + 1][cl] = acc;
           }
+          acc = V::Zero();
         }
       }
       if constexpr (IsInterpreted<EPI>()) {
@@ -1351,15 +1492,14 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
         // body in the instruction cache): each pass updates entry 0 and
         // shifts the rest down, so every index stays constant.
 #pragma unroll 1
-        for (int u = 0; u < kUnroll; ++u) {
-          if (fin[0] && col_ok) {
-            Epilogue<VEC, EPI, kMapped>(r, s_map, kk[0], col, res[0], tv[0],
-                                        av[0], bv[0], H);
+        for (int u = 0; u < U; ++u) {
+          if (act[0] == kActFinish && col_ok) {
+            Epilogue<VEC, EPI, kMapped>(r, s_map, s_key[base + q + u + 1], col,
+                                        res[0], tv[0], av[0], bv[0], H);
           }
 #pragma unroll
-          for (int j = 0; j + 1 < kUnroll; ++j) {
-            fin[j] = fin[j + 1];
-            kk[j] = kk[j + 1];
+          for (int j = 0; j + 1 < U; ++j) {
+            act[j] = act[j + 1];
             res[j] = res[j + 1];
             tv[j] = tv[j + 1];
             av[j] = av[j + 1];
@@ -1383,9 +1523,12 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
         g = V::Add(g, s_part[2 * tt][cl]);
         ended = (inf & kHeadEnds) != 0;
       }
-      const uint32_t key = job == 0 ? s_key[1] : s_key[base + cnt];
+      // A range with a tail is full (or the stream's last), and ends in it.
+      const int64_t left = n - (cb + base);
+      const int cnt = left < R ? static_cast<int>(left) : R;
+      const uint32_t kj = job == 0 ? s_key[1] : s_key[base + cnt];
       if (job == 1 && ended) {
-        if (col_ok) EpilogueLoad<VEC, EPI, kMapped>(r, s_map, key, col, g, H);
+        if (col_ok) EpilogueLoad<VEC, EPI, kMapped>(r, s_map, kj, col, g, H);
       } else if (col_ok) {
         const int64_t slot = job == 1 ? 2 * blk + 1 : 2 * blk;
         V::Store(r.partials + slot * dim + col, g);
@@ -2358,12 +2501,36 @@ int LaunchRtc(const RtcKernels& k, StreamArgs st, RowArgs r, int64_t num_blocks,
   return 0;
 }
 
+// Entries of a sub-group's range. A range of G entries makes blocks of kBlock
+// entries, the most blocks for a short stream. With narrow rows (G < 32) that
+// leaves a sub-group few entries beside its pieces, flags and barriers, so
+// streams with blocks to spare take longer ranges where AnyOrder allows it.
+constexpr int LongRange(int g) { return g < 16 ? 16 : g < 32 ? 32 : g; }
+constexpr int64_t kLongRangeBlocks = 512;
+inline bool UseLongRange(int g, int64_t n) {
+  return LongRange(g) > g &&
+         n >= kLongRangeBlocks * (kBlock / g) * LongRange(g);
+}
+
+template <int G, int VEC, int SRC, int EPI, bool kOneHot, bool kMapped>
+void LaunchReduce(const StreamArgs& st, const RowArgs& r, bool long_range,
+                  dim3 grid, hipStream_t stream) {
+  if constexpr (LongRange(G) > G && AnyOrder<EPI>()) {
+    if (long_range) {
+      hipLaunchKernelGGL(
+          (SegReduce<G, VEC, SRC, EPI, kOneHot, kMapped, LongRange(G)>), grid,
+          dim3(kBlock), 0, stream, st, r);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((SegReduce<G, VEC, SRC, EPI, kOneHot, kMapped, G>), grid,
+                     dim3(kBlock), 0, stream, st, r);
+}
+
 template <int SRC, int EPI, bool kMapped>
 int LaunchSegMapped(const StreamArgs& st, RowArgs r, const SegBuffers& sb,
                     int g, int vec, bool one_hot, const char* reduce_span,
                     const char* finish_span, hipStream_t stream) {
-  constexpr int kWide = EPI == kEpiFwd ? kFwdUnrollWide : kBwdUnrollWide;
-  constexpr int kNarrow = EPI == kEpiFwd ? kFwdUnrollNarrow : kBwdUnrollNarrow;
   r.partials = sb.partials;
   r.block_flags = sb.flags;
   r.block_keys = sb.keys;
@@ -2371,32 +2538,35 @@ int LaunchSegMapped(const StreamArgs& st, RowArgs r, const SegBuffers& sb,
     // A custom program runs compiled for itself when it can (the same
     // kernels with its update inlined), else through the interpreter.
     RtcKernels k{};
-    const int rc = RtcKernelsFor(r.opt.prog, g, vec, SRC,
-                                 one_hot ? kWide : kNarrow, kMapped, &k);
+    const int rc =
+        RtcKernelsFor(r.opt.prog, g, vec, SRC, one_hot, kMapped, &k);
     if (rc == 0) {
       return LaunchRtc(k, st, r, sb.num_blocks, reduce_span, finish_span,
                        stream);
     }
     if (rc != kRtcInterpret) return rc;
   }
-  const dim3 grid(static_cast<uint32_t>(sb.num_blocks));
+  const bool long_range = AnyOrder<EPI>() && UseLongRange(g, st.n);
+  const int64_t num_blocks =
+      long_range ? CeilDiv(st.n, kBlock / g * LongRange(g)) : sb.num_blocks;
+  const dim3 grid(static_cast<uint32_t>(num_blocks));
 #define SCEMB_SEG_CASE(GG, VV)                                                \
   if constexpr (VV == 1 || EPI != kEpiCustom)                                \
   if (g == GG && vec == VV) {                                                \
     int prof = ProfileBegin(reduce_span, stream);                            \
     if (one_hot) {                                                           \
-      hipLaunchKernelGGL((SegReduce<GG, VV, SRC, EPI, kWide, kMapped>), grid, \
-                         dim3(kBlock), 0, stream, st, r);                     \
+      LaunchReduce<GG, VV, SRC, EPI, true, kMapped>(st, r, long_range, grid,  \
+                                                    stream);                  \
     } else {                                                                 \
-      hipLaunchKernelGGL((SegReduce<GG, VV, SRC, EPI, kNarrow, kMapped>),     \
-                         grid, dim3(kBlock), 0, stream, st, r);               \
+      LaunchReduce<GG, VV, SRC, EPI, false, kMapped>(st, r, long_range, grid, \
+                                                     stream);                 \
     }                                                                        \
     ProfileEnd(prof, stream);                                                 \
     SCEMB_LAUNCH_CHECK();                                                     \
     if (r.single_runs) return 0;                                              \
     prof = ProfileBegin(finish_span, stream);                                 \
     hipLaunchKernelGGL((SegFinish<GG, VV, EPI, kMapped>), grid, dim3(kBlock), \
-                       0, stream, sb.num_blocks, r);                          \
+                       0, stream, num_blocks, r);                             \
     ProfileEnd(prof, stream);                                                 \
     SCEMB_LAUNCH_CHECK();                                                     \
     return 0;                                                                 \
@@ -2650,7 +2820,6 @@ int GradImpl(const GradCall& c) {
   r.opt = c.opt;
   r.status = c.status;
   if (c.map != nullptr) r.act = *c.map;
-  r.stream_src = one_hot;
   int g, vec;
   PickLayout(dim,
              Aligned16(c.table) &&
