@@ -226,11 +226,8 @@ __device__ __forceinline__ void RadixScatterBody(
   for (int c = 0; c < kWaveChunks; ++c) {
     const bool active = act[c];
     const uint32_t d = active ? Digit(key[c], shift, mask) : 0u;
-    uint64_t match = __ballot(active);
-    for (int b = 0; b < digit_bits; ++b) {
-      const uint64_t bits = __ballot((d >> b) & 1u);
-      match &= ((d >> b) & 1u) ? bits : ~bits;
-    }
+    // The digit's bits past digit_bits are zero.
+    const uint64_t match = MatchLanes<kMaxDigitBits>(__ballot(active), d, 0);
     // The lowest lane of each digit group bumps the wave's counter; the
     // group reads the count before the bump from it.
     const bool leader = active && (match & lt) == 0;
@@ -393,11 +390,8 @@ __device__ __forceinline__ void BucketLdsPass(
     if (w0 + c * kWave >= w1) break;  // uniform: the wave's span ended
     const bool active = w0 + c * kWave + lane < w1;
     const uint32_t v = (static_cast<uint32_t>(key[c]) >> shift) & mask;
-    uint64_t match = __ballot(active);
-    for (int b = 0; b < bits; ++b) {
-      const uint64_t bb = __ballot((v >> b) & 1u);
-      match &= ((v >> b) & 1u) ? bb : ~bb;
-    }
+    const uint64_t match =
+        MatchLanes<kBucketDigitMax>(__ballot(active), v, 0);
     const bool leader = active && (match & lt) == 0;
     uint32_t before = 0;
     if (leader) {
