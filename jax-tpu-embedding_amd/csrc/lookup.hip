@@ -170,7 +170,7 @@ int GroupByRowInBuckets(const CsrRowSource& src, int64_t n,
       (radix::RadixScatterK<uint32_t, uint64_t, CsrRowSource,
                             radix::ArraySink<uint32_t, uint64_t>>),
       dim3(tiles), dim3(kSortBlock), 0, stream, src, mid, n, n_dev,
-      n_dev_words, lb, mask, hb, tiles, hist, total, false);
+      n_dev_words, lb, mask, tiles, hist, total, false);
   SCEMB_LAUNCH_CHECK();
   const StreamSink sink{b.keys, b.pay, static_cast<uint32_t>(batch)};
   hipLaunchKernelGGL(
@@ -260,13 +260,13 @@ int GroupByRow(const scemb_csr_t* csr, const Geometry& geo, int64_t batch,
             (radix::RadixScatterK<uint32_t, uint64_t, CsrRowSource,
                                   StreamSink>),
             dim3(tiles), dim3(kSortBlock), 0, stream, csr_src, sink, n,
-            csr_end, csr_end_words, shift, mask, pbits, tiles, hist,
+            csr_end, csr_end_words, shift, mask, tiles, hist,
             totals + pass, last);
       } else {
         hipLaunchKernelGGL(
             (radix::RadixScatterK<uint32_t, uint64_t, Arr, StreamSink>),
             dim3(tiles), dim3(kSortBlock), 0, stream, arr, sink, n, taken, 1,
-            shift, mask, pbits, tiles, hist, totals + pass, last);
+            shift, mask, tiles, hist, totals + pass, last);
       }
       SCEMB_LAUNCH_CHECK();
     }

@@ -177,7 +177,7 @@ constexpr int kWaveChunks = kWaveSpan / kWave;      // 8 chunks of 64
 template <typename K, typename V, typename Src, typename Sink>
 __device__ __forceinline__ void RadixScatterBody(
     uint32_t tile_index, Src src, Sink sink, int64_t n, const uint32_t* n_dev,
-    int n_dev_words, int shift, uint32_t mask, int digit_bits, int64_t tiles,
+    int n_dev_words, int shift, uint32_t mask, int64_t tiles,
     const uint32_t* offsets, const uint32_t* total, bool fill_tail) {
   __shared__ uint32_t wave_cnt[kSortWaves][kMaxRadix];
   __shared__ uint32_t global_off[kMaxRadix];  // bucket start (output)
@@ -226,7 +226,7 @@ __device__ __forceinline__ void RadixScatterBody(
   for (int c = 0; c < kWaveChunks; ++c) {
     const bool active = act[c];
     const uint32_t d = active ? Digit(key[c], shift, mask) : 0u;
-    // The digit's bits past digit_bits are zero.
+    // A narrower digit's upper bits are zero.
     const uint64_t match = MatchLanes<kMaxDigitBits>(__ballot(active), d, 0);
     // The lowest lane of each digit group bumps the wave's counter; the
     // group reads the count before the bump from it.
@@ -295,11 +295,11 @@ __device__ __forceinline__ void RadixScatterBody(
 template <typename K, typename V, typename Src, typename Sink>
 __global__ __launch_bounds__(kSortBlock) void RadixScatterK(
     Src src, Sink sink, int64_t n, const uint32_t* n_dev, int n_dev_words,
-    int shift, uint32_t mask, int digit_bits, int64_t tiles, const uint32_t* offsets,
+    int shift, uint32_t mask, int64_t tiles, const uint32_t* offsets,
     const uint32_t* total, bool fill_tail) {
   RadixScatterBody<K, V, Src, Sink>(blockIdx.x, src, sink, n, n_dev,
-                                    n_dev_words, shift, mask, digit_bits,
-                                    tiles, offsets, total, fill_tail);
+                                    n_dev_words, shift, mask, tiles, offsets,
+                                    total, fill_tail);
 }
 
 // RadixScatterK's arguments for a grouped launch (common.h).
@@ -313,7 +313,6 @@ struct RadixScatterArgs {
   int n_dev_words;
   int shift;
   uint32_t mask;
-  int digit_bits;
   int64_t tiles;
   const uint32_t* offsets;
   const uint32_t* total;
@@ -322,8 +321,8 @@ struct RadixScatterArgs {
                              uint32_t) {
     RadixScatterBody<K, V, Src, Sink>(blk, a.src, a.sink, a.n, a.n_dev,
                                       a.n_dev_words, a.shift, a.mask,
-                                      a.digit_bits, a.tiles, a.offsets,
-                                      a.total, a.fill_tail);
+                                      a.tiles, a.offsets, a.total,
+                                      a.fill_tail);
   }
 };
 

@@ -291,7 +291,7 @@ int RadixSortPairs(K* keys, V* vals, K* keys_alt, V* vals_alt, int64_t n,
           (radix::RadixScatterK<K, V, radix::ArraySource<K, V>,
                                 radix::ArraySink<K, V>>),
           dim3(tiles), dim3(kSortBlock), 0, stream, src, sink, n, nullptr, 0,
-          shift, mask, bits, tiles, hist, total, false);
+          shift, mask, tiles, hist, total, false);
       SCEMB_LAUNCH_CHECK();
     }
     K* tk = src_k;
