@@ -2032,13 +2032,26 @@ __global__ __launch_bounds__(kHotTileBlock) void HotTile(StreamArgs st,
   // gradient matrix, copied into LDS by DMA loads (global_load_lds, 16
   // bytes per lane to the wave's LDS base + 16 * lane) while the block
   // reads its runs' ranges; the copy is waited for before the reduction.
-  const bool dma = !kMapped && VEC == 4 &&
-                   (reinterpret_cast<uintptr_t>(r.src) & 15u) == 0;
+  // Through a row map that holds where the tile lies in one block of full,
+  // contiguous rows, as nearly all do; a tile across blocks resolves every
+  // row (batch 131,072, one block of 128 columns: 61 us alone, with every
+  // vector's row looked up in the map; 57 us so).
+  const float* dense = kMapped ? nullptr : r.src + row0 * dim;
+  if (kMapped) {
+    for (int b = 0; b < r.act.n; ++b) {
+      if (row0 >= r.act.first[b] && row0 + rows <= r.act.end[b] &&
+          r.act.stride[b] == dim && r.act.width[b] == dim) {
+        dense = r.act.data[b] + (row0 - r.act.first[b]) * dim;
+      }
+    }
+  }
+  const bool dma = VEC == 4 && dense != nullptr &&
+                   (reinterpret_cast<uintptr_t>(dense) & 15u) == 0;
   bool staged = dma;
   if (dma) {
     constexpr int kChunk = kWave * 16;  // bytes one wave copies at once
     const int64_t bytes = static_cast<int64_t>(rows) * dim * sizeof(float);
-    const char* src = reinterpret_cast<const char*>(r.src + row0 * dim);
+    const char* src = reinterpret_cast<const char*>(dense);
     const int wave = tid / kWave;
     const int lane = tid % kWave;
     for (int64_t c = static_cast<int64_t>(wave) * kChunk; c < bytes;
