@@ -26,8 +26,12 @@ constexpr int kSortBlock = 256;
 constexpr int kSortChunks = 8;
 constexpr int kSortTile = kSortBlock * kSortChunks;
 constexpr int kMaxDigitBits = 8;
-constexpr int kMaxRadix = 1 << kMaxDigitBits;
-constexpr int kSortWaves = kSortBlock / kWave;
+// Passes of a wider digit, for key widths that then take one pass fewer: 512
+// threads and tiles of 4,096, so that a tile still holds eight elements per
+// digit on average (its writes come out bucket by bucket).
+constexpr int kWideBlock = 512;
+constexpr int kWideTile = kWideBlock * kSortChunks;
+constexpr int kWideDigitBits = 9;
 
 template <typename K>
 __device__ __forceinline__ uint32_t Digit(K key, int shift, uint32_t mask) {
@@ -80,17 +84,18 @@ __device__ __forceinline__ int64_t ActiveCount(int64_t n,
 // hist[d * tiles + tile] = elements of digit d in the tile. The positions
 // the source declines go to src.Rejected after all loads are issued.
 // The body of work-group `tile` (RadixHistogramK and grouped launches).
-template <typename K, typename Src>
+template <typename K, typename Src, int kBlk = kSortBlock,
+          int kBits = kMaxDigitBits>
 __device__ __forceinline__ void RadixHistogramBody(
     uint32_t tile_index, Src src, int64_t n, const uint32_t* n_dev,
     int n_dev_words, int shift, uint32_t mask, int64_t tiles, uint32_t* hist) {
-  __shared__ uint32_t h[kMaxRadix];
+  __shared__ uint32_t h[1 << kBits];
   const int radix = static_cast<int>(mask) + 1;
-  for (int d = threadIdx.x; d < radix; d += kSortBlock) h[d] = 0;
+  for (int d = threadIdx.x; d < radix; d += kBlk) h[d] = 0;
   __syncthreads();
   const int64_t m = ActiveCount(n, n_dev, n_dev_words);
   const int64_t tile = tile_index;
-  const int64_t base = tile * kSortTile;
+  const int64_t base = tile * (kBlk * kSortChunks);
   // All of the thread's keys first: the source reads through pointers that
   // the compiler cannot tell apart from the LDS counters, so loads issued
   // between the atomics would each wait for the one before.
@@ -98,7 +103,7 @@ __device__ __forceinline__ void RadixHistogramBody(
   bool act[kSortChunks];
 #pragma unroll
   for (int c = 0; c < kSortChunks; ++c) {
-    const int64_t i = base + c * kSortBlock + threadIdx.x;
+    const int64_t i = base + c * kBlk + threadIdx.x;
     act[c] = i < m && src.LoadKey(i, &keys[c]);
   }
 #pragma unroll
@@ -123,11 +128,11 @@ __device__ __forceinline__ void RadixHistogramBody(
   }
 #pragma unroll
   for (int c = 0; c < kSortChunks; ++c) {
-    const int64_t i = base + c * kSortBlock + threadIdx.x;
+    const int64_t i = base + c * kBlk + threadIdx.x;
     if (i < m && !act[c]) src.Rejected(i);
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < radix; d += kSortBlock) {
+  for (int d = threadIdx.x; d < radix; d += kBlk) {
     hist[static_cast<int64_t>(d) * tiles + tile] = h[d];
   }
 }
@@ -141,9 +146,10 @@ __global__ __launch_bounds__(kSortBlock) void RadixHistogramK(
 }
 
 // RadixHistogramK's arguments for a grouped launch (common.h).
-template <typename K, typename Src>
+template <typename K, typename Src, int kBlk = kSortBlock,
+          int kBits = kMaxDigitBits>
 struct RadixHistogramArgs {
-  static constexpr int kBlock = kSortBlock;
+  static constexpr int kBlock = kBlk;
   Src src;
   int64_t n;
   const uint32_t* n_dev;
@@ -154,8 +160,9 @@ struct RadixHistogramArgs {
   uint32_t* hist;
   __device__ static void Run(const RadixHistogramArgs& a, uint32_t blk,
                              uint32_t) {
-    RadixHistogramBody<K, Src>(blk, a.src, a.n, a.n_dev, a.n_dev_words,
-                               a.shift, a.mask, a.tiles, a.hist);
+    RadixHistogramBody<K, Src, kBlk, kBits>(blk, a.src, a.n, a.n_dev,
+                                            a.n_dev_words, a.shift, a.mask,
+                                            a.tiles, a.hist);
   }
 };
 
@@ -171,40 +178,44 @@ struct RadixHistogramArgs {
 // One scan over (wave, digit) then gives every element its place in the
 // tile, which is staged in LDS bucket by bucket and written out so that
 // consecutive threads write consecutive output positions.
-constexpr int kWaveSpan = kSortTile / kSortWaves;   // 512 positions
-constexpr int kWaveChunks = kWaveSpan / kWave;      // 8 chunks of 64
+constexpr int kWaveChunks = kSortChunks;            // chunks of 64
+constexpr int kWaveSpan = kWaveChunks * kWave;      // 512 positions
 
-template <typename K, typename V, typename Src, typename Sink>
+template <typename K, typename V, typename Src, typename Sink,
+          int kBlk = kSortBlock, int kBits = kMaxDigitBits>
 __device__ __forceinline__ void RadixScatterBody(
     uint32_t tile_index, Src src, Sink sink, int64_t n, const uint32_t* n_dev,
     int n_dev_words, int shift, uint32_t mask, int64_t tiles,
     const uint32_t* offsets, const uint32_t* total, bool fill_tail) {
-  __shared__ uint32_t wave_cnt[kSortWaves][kMaxRadix];
-  __shared__ uint32_t global_off[kMaxRadix];  // bucket start (output)
-  __shared__ uint32_t tile_off[kMaxRadix];    // bucket start (tile)
-  __shared__ uint32_t scan_tmp[kSortBlock / kWave + 1];
-  __shared__ K s_keys[kSortTile];
-  __shared__ V s_vals[kSortTile];
+  constexpr int kTile = kBlk * kSortChunks;
+  constexpr int kWaves = kBlk / kWave;
+  constexpr int kRadix = 1 << kBits;
+  __shared__ uint16_t wave_cnt[kWaves][kRadix];  // at most kTile
+  __shared__ uint32_t global_off[kRadix];  // bucket start (output)
+  __shared__ uint32_t tile_off[kRadix];    // bucket start (tile)
+  __shared__ uint32_t scan_tmp[kWaves + 1];
+  __shared__ K s_keys[kTile];
+  __shared__ V s_vals[kTile];
   const int t = threadIdx.x;
   const int wave = t / kWave;
   const int lane = t % kWave;
   const int radix = static_cast<int>(mask) + 1;
   const int64_t blk = tile_index;
-  const int64_t base = blk * kSortTile;
+  const int64_t base = blk * kTile;
   if (fill_tail) {
     const int64_t taken = static_cast<int64_t>(*total);
-    for (int64_t i = base + t; i < base + kSortTile && i < n;
-         i += kSortBlock) {
+    for (int64_t i = base + t; i < base + kTile && i < n;
+         i += kBlk) {
       if (i >= taken) sink.Fill(i);
     }
   }
   const int64_t m = ActiveCount(n, n_dev, n_dev_words);
   if (base >= m) return;  // uniform: the whole block
   const int tile_n =
-      static_cast<int>(m - base < kSortTile ? m - base : kSortTile);
-  for (int b = t; b < radix; b += kSortBlock) {
+      static_cast<int>(m - base < kTile ? m - base : kTile);
+  for (int b = t; b < radix; b += kBlk) {
 #pragma unroll
-    for (int w = 0; w < kSortWaves; ++w) wave_cnt[w][b] = 0;
+    for (int w = 0; w < kWaves; ++w) wave_cnt[w][b] = 0;
     global_off[b] = offsets[static_cast<int64_t>(b) * tiles + blk];
   }
   __syncthreads();
@@ -227,14 +238,15 @@ __device__ __forceinline__ void RadixScatterBody(
     const bool active = act[c];
     const uint32_t d = active ? Digit(key[c], shift, mask) : 0u;
     // A narrower digit's upper bits are zero.
-    const uint64_t match = MatchLanes<kMaxDigitBits>(__ballot(active), d, 0);
+    const uint64_t match = MatchLanes<kBits>(__ballot(active), d, 0);
     // The lowest lane of each digit group bumps the wave's counter; the
     // group reads the count before the bump from it.
     const bool leader = active && (match & lt) == 0;
     uint32_t before = 0;
     if (leader) {
       before = wave_cnt[wave][d];
-      wave_cnt[wave][d] = before + static_cast<uint32_t>(__popcll(match));
+      wave_cnt[wave][d] = static_cast<uint16_t>(
+          before + static_cast<uint32_t>(__popcll(match)));
     }
     const int src_lane = active ? __ffsll(static_cast<long long>(match)) - 1
                                 : lane;
@@ -246,17 +258,17 @@ __device__ __forceinline__ void RadixScatterBody(
   __syncthreads();
   // Per digit: the waves' counts become exclusive wave bases, their sum the
   // tile's bucket size, scanned over digits into the tile offsets.
-  constexpr int kRounds = kMaxRadix / kSortBlock;
+  constexpr int kRounds = (kRadix + kBlk - 1) / kBlk;
   uint32_t cnt[kRounds];
 #pragma unroll
   for (int k = 0; k < kRounds; ++k) {
-    const int d = t + k * kSortBlock;
+    const int d = t + k * kBlk;
     uint32_t r = 0;
     if (d < radix) {
 #pragma unroll
-      for (int w = 0; w < kSortWaves; ++w) {
+      for (int w = 0; w < kWaves; ++w) {
         const uint32_t c = wave_cnt[w][d];
-        wave_cnt[w][d] = r;
+        wave_cnt[w][d] = static_cast<uint16_t>(r);
         r += c;
       }
     }
@@ -266,9 +278,9 @@ __device__ __forceinline__ void RadixScatterBody(
 #pragma unroll
   for (int k = 0; k < kRounds; ++k) {
     uint32_t round_total;
-    const uint32_t ex = BlockExclusiveScan<uint32_t, kSortBlock>(
+    const uint32_t ex = BlockExclusiveScan<uint32_t, kBlk>(
         cnt[k], scan_tmp, &round_total);
-    const int d = t + k * kSortBlock;
+    const int d = t + k * kBlk;
     if (d < radix) tile_off[d] = round_base + ex;
     round_base += round_total;
     __syncthreads();
@@ -284,7 +296,7 @@ __device__ __forceinline__ void RadixScatterBody(
   }
   __syncthreads();
   // Element j of digit d goes to global_off[d] + (j - tile_off[d]).
-  for (int j = t; j < tile_taken; j += kSortBlock) {
+  for (int j = t; j < tile_taken; j += kBlk) {
     const K k = s_keys[j];
     const uint32_t d = Digit(k, shift, mask);
     sink.Store(global_off[d] + (static_cast<uint32_t>(j) - tile_off[d]), k,
@@ -303,9 +315,10 @@ __global__ __launch_bounds__(kSortBlock) void RadixScatterK(
 }
 
 // RadixScatterK's arguments for a grouped launch (common.h).
-template <typename K, typename V, typename Src, typename Sink>
+template <typename K, typename V, typename Src, typename Sink,
+          int kBlk = kSortBlock, int kBits = kMaxDigitBits>
 struct RadixScatterArgs {
-  static constexpr int kBlock = kSortBlock;
+  static constexpr int kBlock = kBlk;
   Src src;
   Sink sink;
   int64_t n;
@@ -319,10 +332,9 @@ struct RadixScatterArgs {
   bool fill_tail;
   __device__ static void Run(const RadixScatterArgs& a, uint32_t blk,
                              uint32_t) {
-    RadixScatterBody<K, V, Src, Sink>(blk, a.src, a.sink, a.n, a.n_dev,
-                                      a.n_dev_words, a.shift, a.mask,
-                                      a.tiles, a.offsets, a.total,
-                                      a.fill_tail);
+    RadixScatterBody<K, V, Src, Sink, kBlk, kBits>(
+        blk, a.src, a.sink, a.n, a.n_dev, a.n_dev_words, a.shift, a.mask,
+        a.tiles, a.offsets, a.total, a.fill_tail);
   }
 };
 
@@ -632,9 +644,9 @@ struct DigitPlan {
   int passes;
   int digit;
 };
-inline DigitPlan PlanDigits(int span) {
+inline DigitPlan PlanDigits(int span, int max_bits = kMaxDigitBits) {
   DigitPlan p;
-  p.passes = span <= 0 ? 0 : (span + kMaxDigitBits - 1) / kMaxDigitBits;
+  p.passes = span <= 0 ? 0 : (span + max_bits - 1) / max_bits;
   p.digit = p.passes == 0 ? 0 : (span + p.passes - 1) / p.passes;
   return p;
 }

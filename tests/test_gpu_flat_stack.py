@@ -1,6 +1,7 @@
 """The preprocessing of a stack on one device and one SparseCore, whose sort
 reads the sample view and writes the CSR (preprocess.hip, UniqueStack::flat):
-sizes around its extraction blocks, view and counting work-groups, inputs of
+sizes around its extraction blocks, view and counting work-groups, key widths
+around its digits, inputs of
 one id, of copies only, of ids outside the table only, and a static buffer
 smaller than the input (the general path). The route that merges after the
 sort gives the same CSR, stats and views bit for bit."""
@@ -41,3 +42,16 @@ def test_nothing_left_or_little_room(what):
   limit = 512 if what == "small buffer" else 1 << 14
   specs = _specs([("a", 50)], len(lens), "sum", 1, 1, limit)
   _compare(what, feats, None, specs)
+
+
+@pytest.mark.parametrize("bits", [8, 9, 10, 16, 17, 18, 19, 24, 25, 27, 28])
+def test_key_widths_around_the_digits(bits):
+  """Key widths where one pass of wider digits replaces two, and their
+  neighbours, over more than one of either tile."""
+  if not torch.cuda.is_available():
+    pytest.skip("no GPU")
+  rng = np.random.default_rng(bits)
+  lens = rng.integers(0, 20, size=1000)
+  specs = _specs([("a", 2**bits)], len(lens), "sum", 1, 1, 1 << 16)
+  feats = [_ragged(rng, lens, 2**bits)]
+  _compare(bits, feats, None, specs)
