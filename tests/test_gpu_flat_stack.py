@@ -1,6 +1,7 @@
 """The preprocessing of a stack on one device and one SparseCore, whose sort
 reads the sample view and writes the CSR (preprocess.hip, UniqueStack::flat):
-sizes around its extraction blocks, view and counting work-groups, key widths
+sizes around its extraction blocks, its work-groups and the one work-group of
+small stacks (16,384 ids), key widths
 around its digits, inputs of
 one id, of copies only, of ids outside the table only, and a static buffer
 smaller than the input (the general path). The route that merges after the
