@@ -191,10 +191,16 @@ __global__ __launch_bounds__(A::kBlock) void GroupedKernel(Group<A> g) {
   A::Run(g.a[p], blockIdx.x - g.first[p], g.first[p + 1] - g.first[p]);
 }
 
+// One problem alone, whose arguments are an eighth as long.
+template <typename A>
+__global__ __launch_bounds__(A::kBlock) void SingleKernel(A a) {
+  A::Run(a, blockIdx.x, gridDim.x);
+}
+
 #ifndef __HIPCC_RTC__
 // Enqueues GroupedKernel<A> over problems i with args[i] and blocks[i]
-// work-groups, at most kMaxGroup per launch; problems of no blocks are left
-// out.
+// work-groups, at most kMaxGroup per launch (SingleKernel<A> for one); problems
+// of no blocks are left out.
 template <typename A>
 int LaunchGrouped(const A* args, const int64_t* blocks, int n,
                   hipStream_t stream) {
@@ -209,8 +215,14 @@ int LaunchGrouped(const A* args, const int64_t* blocks, int n,
     if (!last && b <= 0) continue;
     if (g.n > 0 && (last || g.n == kMaxGroup || total + b > 0xffffffffll)) {
       g.first[g.n] = static_cast<uint32_t>(total);
-      hipLaunchKernelGGL(GroupedKernel<A>, dim3(static_cast<uint32_t>(total)),
-                         dim3(A::kBlock), 0, stream, g);
+      const dim3 grid(static_cast<uint32_t>(total));
+      if (g.n == 1) {
+        hipLaunchKernelGGL(SingleKernel<A>, grid, dim3(A::kBlock), 0, stream,
+                           g.a[0]);
+      } else {
+        hipLaunchKernelGGL(GroupedKernel<A>, grid, dim3(A::kBlock), 0, stream,
+                           g);
+      }
       SCEMB_LAUNCH_CHECK();
       g.n = 0;
       total = 0;
