@@ -489,10 +489,20 @@ def check_status_word(word, what: str) -> None:
 # ---------------------------------------------------------------------------
 
 
-def torch():
-  import torch as _torch  # pylint: disable=g-import-not-at-top
+# What a call asks of the runtime, apart from its launches, is most of a small
+# call's time: torch is imported once, device objects are made once per index
+# and the current stream's handle is read without a stream object (a small
+# training step asks for it seven times, a device a dozen).
+_torch_module = None
 
-  return _torch
+
+def torch():
+  global _torch_module
+  if _torch_module is None:
+    import torch as _torch  # pylint: disable=g-import-not-at-top
+
+    _torch_module = _torch
+  return _torch_module
 
 
 _gpu_seen = False
@@ -616,14 +626,29 @@ def run_per_stack(names, fn, width=None) -> dict:
   return out
 
 
-def stream_handle() -> int:
+def _raw_stream(index: int) -> int:
+  """The handle of device `index`'s current stream."""
   t = torch()
-  return t.cuda.current_stream().cuda_stream
+  raw = getattr(t._C, "_cuda_getCurrentRawStream", None)  # pylint: disable=protected-access
+  if raw is None:
+    return t.cuda.current_stream(index).cuda_stream
+  return raw(index)
+
+
+def stream_handle() -> int:
+  return _raw_stream(torch().cuda.current_device())
+
+
+_devices = {}
 
 
 def device() -> "torch.device":
   t = require_gpu()
-  return t.device("cuda", t.cuda.current_device())
+  index = t.cuda.current_device()
+  dev = _devices.get(index)
+  if dev is None:
+    dev = _devices[index] = t.device("cuda", index)
+  return dev
 
 
 def as_device_tensor(x, dtype, dev=None):
@@ -633,7 +658,7 @@ def as_device_tensor(x, dtype, dev=None):
   if isinstance(x, t.Tensor):
     if x.device != dev or x.dtype != dtype:
       x = x.to(device=dev, dtype=dtype)
-    return x.contiguous()
+    return x if x.is_contiguous() else x.contiguous()
   arr = np.asarray(x)
   np_dtype = {t.int32: np.int32, t.int64: np.int64,
               t.float32: np.float32}[dtype]
@@ -793,14 +818,13 @@ class _Workspace:
     on it is done."""
     t = torch()
     dev = device()
-    if stream is None:
-      stream = t.cuda.current_stream(dev)
-    key = (dev.index, stream.cuda_stream)
+    key = (dev.index, _raw_stream(dev.index) if stream is None else
+           stream.cuda_stream)
     buf = self._buf.get(key)
     if buf is None or buf.numel() < nbytes:
       if buf is not None and key in self._captured:
         self._retired.append(buf)
-      with t.cuda.stream(stream):
+      with t.cuda.stream(stream or t.cuda.current_stream(dev)):
         buf = t.empty(max(int(nbytes * 1.25), 1 << 20), dtype=t.uint8,
                       device=dev)
       self._buf[key] = buf

@@ -91,10 +91,19 @@ def tree_structure(tree):
 
 
 def tree_map(fn: Callable, tree, *rest) -> Any:
+  if not rest and _flat_leaves(tree):
+    return type(tree)([fn(x) for x in tree])
   leaves, treedef = tree_flatten(tree)
   others = [tree_flatten(r)[0] for r in rest]
   return tree_unflatten(treedef,
                         [fn(*xs) for xs in zip(leaves, *others)])
+
+
+def same_paths(a, b) -> bool:
+  """leaf_paths(a) == leaf_paths(b)."""
+  if _flat_leaves(a) and _flat_leaves(b):
+    return len(a) == len(b)
+  return leaf_paths(a) == leaf_paths(b)
 
 
 def leaf_paths(tree) -> list:

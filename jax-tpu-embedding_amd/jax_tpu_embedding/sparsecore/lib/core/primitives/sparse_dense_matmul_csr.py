@@ -40,7 +40,9 @@ def resolve_minibatches(num_minibatches, enable_minibatching: bool) -> int:
   sparse_dense_matmul_csr.py:171-192 of the reference)."""
   if not enable_minibatching:
     if isinstance(num_minibatches, (int, np.integer, np.ndarray)):
-      if int(np.asarray(num_minibatches).reshape(())) != 1:
+      if (int(np.asarray(num_minibatches).reshape(()))
+          if isinstance(num_minibatches, np.ndarray) else
+          num_minibatches) != 1:
         raise ValueError("num_minibatches must be 1 without minibatching")
     return 0
   if hasattr(num_minibatches, "item") and not isinstance(

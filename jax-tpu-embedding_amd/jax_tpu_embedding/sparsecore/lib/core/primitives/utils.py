@@ -22,6 +22,11 @@ _NP_OF = {
 }
 
 
+# numpy scalar type of each dtype object seen (torch's and numpy's): the
+# operand checks of one call ask for a dozen.
+_TYPE_OF = {}
+
+
 def _dtype(x):
   # Python scalars are weakly typed (JAX's default 32-bit mode): int -> int32,
   # float -> float32.
@@ -33,10 +38,14 @@ def _dtype(x):
     return np.float32
   if hasattr(x, "dtype"):
     d = x.dtype
-    s = str(d)
-    if s.startswith("torch."):
-      return _NP_OF.get(s, s)
-    return np.dtype(d).type
+    found = _TYPE_OF.get(d)
+    if found is None:
+      s = str(d)
+      found = (_NP_OF.get(s, s) if s.startswith("torch.") else
+               np.dtype(d).type)
+      if len(_TYPE_OF) < 64:
+        _TYPE_OF[d] = found
+    return found
   return np.asarray(x).dtype.type
 
 
@@ -94,9 +103,9 @@ def validate_abstract_eval_params(
              "num_minibatches_per_physical_sparse_core")
   if activations_grad is not None:
     ensure_dim(activations_grad, (1, 2), "activations_grad")
-  if (_shape(lhs_local_sample_ids) != _shape(lhs_local_embedding_ids) or
-      _shape(lhs_gains) != _shape(lhs_local_embedding_ids) or
-      len(_shape(lhs_local_sample_ids)) != 1):
+  entries = _shape(lhs_local_embedding_ids)
+  if (len(entries) != 1 or _shape(lhs_local_sample_ids) != entries or
+      _shape(lhs_gains) != entries):
     raise ValueError(
         "LHS sample IDs, embedding IDs, and gains must all have "
         "equal rank 1 shapes, got shapes "

@@ -39,7 +39,7 @@ get_default_limits = table_stacking.get_default_limits
 
 
 def _assert_same_structure(a, b, a_name="a", b_name="b"):
-  if _tree.leaf_paths(a) != _tree.leaf_paths(b):
+  if not _tree.same_paths(a, b):
     raise ValueError(f"Pytree structures of {a_name} and {b_name} do not "
                      "match.")
 
@@ -175,13 +175,16 @@ def get_table_specs(feature_specs):
 
 
 def get_stacked_table_specs(feature_specs):
-  _verify_feature_specs(feature_specs)
   leaves = _tree.tree_leaves(feature_specs)
-  if any(not fs.table_spec.is_stacked() for fs in leaves):
-    raise ValueError(
-        "embedding.prepare_feature_specs_for_training was not called")
-  return {fs.table_spec.stacked_table_spec.stack_name:
-          fs.table_spec.stacked_table_spec for fs in leaves}
+  _verify_feature_specs(leaves)
+  out = {}
+  for fs in leaves:
+    if not fs.table_spec.is_stacked():
+      raise ValueError(
+          "embedding.prepare_feature_specs_for_training was not called")
+    stacked = fs.table_spec.stacked_table_spec
+    out[stacked.stack_name] = stacked
+  return out
 
 
 def prepare_feature_specs_for_training(feature_specs, global_device_count: int,
