@@ -744,9 +744,11 @@ def tpu_sparse_dense_matmul(preprocessed_inputs, embedding_variables,
     return act, fused
 
   # Independent stacks of different widths run concurrently (one side
-  # stream per width); a quantized stack is refused inside its call.
+  # stream per width) when they are large; a quantized stack is refused
+  # inside its call.
   results = _native.run_per_stack(
-      stacked.keys(), lookup, lambda n: stacked[n].stack_embedding_dim)
+      stacked.keys(), lookup, lambda n: stacked[n].stack_embedding_dim,
+      lambda n: _row_bytes(stacked[n], eid[n], counts.get(n)))
   acts = {}
   for name in stacked:
     acts[name], fused = results[name]
@@ -763,6 +765,16 @@ def tpu_sparse_dense_matmul(preprocessed_inputs, embedding_variables,
         use_activation_unstack_primitive)
     per_feature.update({fs.name: a for fs, a in zip(rest, unstacked)})
   return _tree.tree_map(lambda fs: per_feature[fs.name], feature_specs)
+
+
+def _row_bytes(spec, embedding_ids, num_entries) -> int:
+  """About how many bytes of rows a stack's lookup or update moves: a row per
+  CSR entry (`num_entries`, or the buffer's positions while it is not known)
+  and one per sample."""
+  entries = num_entries or (embedding_ids.numel()
+                            if hasattr(embedding_ids, "numel") else
+                            np.size(embedding_ids))
+  return 4 * spec.stack_embedding_dim * (entries + spec.total_sample_count)
 
 
 def _resolve_scalar_minibatches(val):
@@ -941,9 +953,12 @@ def tpu_sparse_dense_matmul_grad(activation_gradients, preprocessed_inputs,
     # (with their slot type), a plain (table, *slots) tuple stays a tuple.
     return _tree.tree_unflatten(treedef, list(res))
 
-  # Independent stacks of different widths update concurrently.
+  # Independent stacks of different widths update concurrently when they are
+  # large.
+  counts = getattr(preprocessed_inputs, "csr_num_entries", None) or {}
   results = _native.run_per_stack(
-      stacked.keys(), update, lambda n: stacked[n].stack_embedding_dim)
+      stacked.keys(), update, lambda n: stacked[n].stack_embedding_dim,
+      lambda n: _row_bytes(stacked[n], eid[n], counts.get(n)))
   return {name: results[name] for name in stacked}
 
 
