@@ -451,7 +451,7 @@ int ForwardImpl(const scemb_csr_t* csr, const scemb_sample_view_t* view,
                                         : csr->num_entries;
   const int64_t entries = hint > 0 && hint < st.n ? hint : st.n;
   const bool one_hot = entries <= kOneHotMaxEntriesPerRow * batch;
-  return LaunchSeg<kSrcSorted, kEpiFwd>(st, r, sb, g, vec, one_hot,
+  return LaunchSeg<kSrcSorted, kEpiFwd>(st, r, sb, entries, g, vec, one_hot,
                                         map != nullptr, "fwd_reduce",
                                         "fwd_finish", stream);
 }

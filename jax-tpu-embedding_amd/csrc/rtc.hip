@@ -185,7 +185,7 @@ Entry Compile(const DevProgram& p, const std::string& arch, int g, int vec,
   const std::string reduce_expr =
       "&scemb::SegReduce<" + layout + ", " + std::to_string(src) + ", " +
       std::to_string(kEpiRtc) + ", " + (one_hot ? "true" : "false") + ", " + m +
-      ", " + std::to_string(g) + ">";
+      ">";
   const std::string finish_expr = "&scemb::SegFinish<" + layout + ", " +
                                   std::to_string(kEpiRtc) + ", " + m + ">";
   hiprtcProgram prog;

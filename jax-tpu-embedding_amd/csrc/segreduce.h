@@ -197,18 +197,30 @@ namespace {
 
 constexpr int kBlock = 256;  // threads per block; entries per hot-run mark
 
-// Whether rows are summed with fused multiply-adds, in ranges of any length:
-// the lookup. The updates keep the order of one multiply and one add per
-// entry in ranges of G, which every update shares (a custom program's result
-// equals the built-in optimizer's bit for bit). It also keeps the last bits of
-// hot rows where they count: such a row adds up 1e5 gradients that nearly
+// Whether rows are summed with fused multiply-adds, and in ranges of two
+// lengths: the lookup. The updates multiply and add, in ranges of G. Built-in,
+// compiled and interpreted updates are all this file's templates, so they
+// would agree in either form; what another order of the sums costs shows in
+// the optimizers with slots: a hot row adds up 1e5 gradients that nearly
 // cancel, and where that leaves a sum near zero, Adagrad's square root turned
-// another order of it into 1e-6 of the size of a later lookup's columns. Of
-// the update of two weighted multi-hot stacks (4.3M entries, 64 columns, SGD)
-// it costs 449 us against 412.
+// another order of it into 1e-6 of the size of a later lookup's columns. That
+// does not hold for SGD, whose update of two weighted multi-hot stacks (4.3M
+// entries, 64 columns) took 412 us fused against 449.
 template <int EPI>
-__host__ __device__ constexpr bool AnyOrder() {
+__host__ __device__ constexpr bool Fuses() {
   return EPI == kEpiFwd;
+}
+
+// The longer of the two lengths that a sub-group's range of entries can have;
+// the shorter is G, which makes the most blocks. G entries of narrow rows
+// (G < 32) leave a sub-group little beside its pieces, flags and barriers.
+// Which one a call takes (TakesLong) changes its speed alone: both add up
+// pieces of G entries, pieces into ranges of 2 * G, those into kBlock entries
+// and these, in pairs, over blocks. (With one running sum over a long range
+// the lookup of two weighted stacks of 64 columns was 5% less exact.)
+template <int EPI>
+__host__ __device__ constexpr int LongRange(int g) {
+  return Fuses<EPI>() && g < 32 ? 2 * g : g;
 }
 
 // Entries whose rows a sub-group loads together (memory-level parallelism;
@@ -1187,17 +1199,24 @@ __device__ __forceinline__ uint32_t FetchCold(const StreamArgs& s, bool hot,
 // instructions to load 16 bytes a lane and add them. So the thread that
 // stages an entry works them out once, and a step is one 16-byte LDS read,
 // one 64-bit add, the load and four fused multiply-adds.
-template <int G, int VEC, int SRC, int EPI, bool kOneHot, bool kMapped, int R>
+template <int G, int VEC, int SRC, int EPI, bool kOneHot, bool kMapped,
+          int R = G>
 __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
   using V = Vec<VEC>;
   using T = typename V::T;
-  constexpr int P = kBlock / G;
+  constexpr int P = kBlock / G;                // sub-groups
   constexpr int kSpan = P * R;                 // entries per block
+  // Sub-groups whose pieces of a run are added up before they join the rest:
+  // those of one long range where ranges are of G, else those of kBlock
+  // entries (as SegFinish adds up the others' blocks in pairs).
+  constexpr bool kTwoLengths = LongRange<EPI>(G) > G;
+  constexpr int kFold = !kTwoLengths ? P : R == G ? 2 : P / 2;
   constexpr int kWaveSpan = kWave / G * R;     // entries per wave
   constexpr int kChunks = kWaveSpan / kWave;   // entries per thread, staged
   constexpr int kUnroll = Unroll<EPI, kOneHot>();
   constexpr int U = kUnroll < R ? kUnroll : R;
   static_assert(R >= G && R <= kWave && kWave % R == 0 && R % U == 0, "range");
+  static_assert(G % U == 0 || U % G == 0, "pieces");
   // Gathered rows read about once (one-hot batches): nontemporal loads.
   constexpr bool kStreamSrc = EPI != kEpiFwd && kOneHot;
   __shared__ uint32_t s_key[kSpan + 2];  // [0]: entry before, last: after
@@ -1240,15 +1259,10 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
   // Entries of hot runs read as outside any run; a block of nothing else
   // has no work.
   const bool hot = SRC == kSrcCsr && st.hot_head != nullptr;
-  if (hot) {
-    bool cold = false;
-    for (int64_t b = cb / kBlock; b < (cb + kSpan) / kBlock && b * kBlock < n;
-         ++b) {
-      int lead, trail;
-      HotSpan(st, b, &lead, &trail);
-      cold = cold || lead < trail;
-    }
-    if (!cold) {
+  if (hot) {  // an update: blocks of kBlock entries
+    int lead, trail;
+    HotSpan(st, blk, &lead, &trail);
+    if (lead >= trail) {
       if (tid == 0) r.block_flags[blk] = 0;
       return;
     }
@@ -1425,6 +1439,7 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
     // Lanes past the last column read along with the first.
     const int64_t lcol = col_ok ? col : 0;
     T acc = V::Zero();
+    T sum = V::Zero();  // R > G: the run's pieces of G entries before acc
     for (int q = range_lo; q < range_hi; q += U) {
       T v[U];
       T tv[U];
@@ -1464,9 +1479,17 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        acc = AnyOrder<EPI>() ? V::Fused(acc, gn[u], v[u])
-                              : V::Fma(acc, gn[u], v[u]);
+        if (R > G && (U > G ? u % G == 0 : u == 0 && q % G == 0)) {
+          sum = V::Add(sum, acc);
+          acc = V::Zero();
+        }
+        acc = Fuses<EPI>() ? V::Fused(acc, gn[u], v[u])
+                           : V::Fma(acc, gn[u], v[u]);
         if (act[u] != kActNone) {
+          if (R > G) {
+            acc = V::Add(sum, acc);
+            sum = V::Zero();
+          }
           if (act[u] == kActFinish) {
             if constexpr (IsInterpreted<EPI>()) {
               res[u] = acc;  // updated below
@@ -1516,13 +1539,19 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
           job == 0 ? (sub == 0 && (info & kHasHead)) : (info & kHasTail) != 0;
       if (!active) continue;
       T g = s_part[job == 0 ? 0 : 2 * sub + 1][cl];
+      T before = V::Zero();
       bool ended = job == 0 && (info & kHeadEnds);
       for (int tt = sub + 1; !ended && tt < P; ++tt) {
         const uint32_t inf = s_info[tt];
         if (!(inf & kHasHead)) break;
+        if (kTwoLengths && tt % kFold == 0) {
+          before = V::Add(before, g);
+          g = V::Zero();
+        }
         g = V::Add(g, s_part[2 * tt][cl]);
         ended = (inf & kHeadEnds) != 0;
       }
+      if (kTwoLengths) g = V::Add(before, g);
       // A range with a tail is full (or the stream's last), and ends in it.
       const int64_t left = n - (cb + base);
       const int cnt = left < R ? static_cast<int>(left) : R;
@@ -1541,8 +1570,9 @@ __global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
 // Runs that cross blocks: the block where such a run starts (kFlagOwner)
 // finds the block where it ends (the next kFlagHeadEnd; every block between
 // is kFlagMiddle), adds the partial rows in block order and applies the
-// epilogue once.
-template <int G, int VEC, int EPI, bool kMapped>
+// epilogue once. kPairs: blocks 2t and 2t + 1 of a run are added first, as the
+// one block of long ranges does that holds their entries.
+template <int G, int VEC, int EPI, bool kMapped, bool kPairs = false>
 __global__ __launch_bounds__(kBlock) void SegFinish(int64_t num_blocks,
                                                     RowArgs r) {
   using V = Vec<VEC>;
@@ -1592,14 +1622,30 @@ __global__ __launch_bounds__(kBlock) void SegFinish(int64_t num_blocks,
     }
     return;
   }
-  const int64_t m = c1 - blk + 1;  // partial rows: 2*blk+1, then 2*(blk+q)
+  // Partial rows 2*blk+1, then 2*(blk+q).
+  const int64_t m = kPairs ? c1 / 2 - blk / 2 + 1 : c1 - blk + 1;
   const Hyper H = LoadHyper<EPI>(r.opt);
   const int64_t dim = r.dim;
   for (int64_t col0 = 0; col0 < dim; col0 += static_cast<int64_t>(G) * VEC) {
     const int64_t col = col0 + static_cast<int64_t>(cl) * VEC;
     const bool col_ok = col < dim;
     T acc = V::Zero();
-    if (col_ok) {
+    if (kPairs && col_ok) {
+      for (int64_t q = sub; q < m; q += P) {
+        const int64_t b1 = (blk / 2 + q) * 2 + 1;
+        T p = V::Zero();
+        if (b1 > blk) {
+          p = V::Load(r.partials +
+                      (b1 - 1 == blk ? 2 * blk + 1 : 2 * (b1 - 1)) * dim + col);
+        }
+        if (b1 <= c1) {
+          p = V::Add(p, V::Load(r.partials +
+                                (b1 == blk ? 2 * blk + 1 : 2 * b1) * dim +
+                                col));
+        }
+        acc = V::Add(acc, p);
+      }
+    } else if (col_ok) {
       int64_t q = sub;
       for (; q + 3 * P < m; q += 4 * P) {
         const T p0 = V::Load(r.partials +
@@ -2514,36 +2560,71 @@ int LaunchRtc(const RtcKernels& k, StreamArgs st, RowArgs r, int64_t num_blocks,
   return 0;
 }
 
-// Entries of a sub-group's range. A range of G entries makes blocks of kBlock
-// entries, the most blocks for a short stream. With narrow rows (G < 32) that
-// leaves a sub-group few entries beside its pieces, flags and barriers, so
-// streams with blocks to spare take longer ranges where AnyOrder allows it.
-constexpr int LongRange(int g) { return g < 16 ? 16 : g < 32 ? 32 : g; }
-constexpr int64_t kLongRangeBlocks = 512;
-inline bool UseLongRange(int g, int64_t n) {
-  return LongRange(g) > g &&
-         n >= kLongRangeBlocks * (kBlock / g) * LongRange(g);
+template <int G, int VEC, int SRC, int EPI, bool kMapped, int R, bool kPairs>
+int LaunchRanges(const StreamArgs& st, const RowArgs& r, bool one_hot,
+                 const char* reduce_span, const char* finish_span,
+                 hipStream_t stream) {
+  const int64_t num_blocks = CeilDiv(st.n, kBlock / G * R);
+  const dim3 grid(static_cast<uint32_t>(num_blocks));
+  int prof = ProfileBegin(reduce_span, stream);
+  if (one_hot) {
+    hipLaunchKernelGGL((SegReduce<G, VEC, SRC, EPI, true, kMapped, R>), grid,
+                       dim3(kBlock), 0, stream, st, r);
+  } else {
+    hipLaunchKernelGGL((SegReduce<G, VEC, SRC, EPI, false, kMapped, R>), grid,
+                       dim3(kBlock), 0, stream, st, r);
+  }
+  ProfileEnd(prof, stream);
+  SCEMB_LAUNCH_CHECK();
+  if (r.single_runs) return 0;
+  prof = ProfileBegin(finish_span, stream);
+  hipLaunchKernelGGL((SegFinish<G, VEC, EPI, kMapped, kPairs>), grid,
+                     dim3(kBlock), 0, stream, num_blocks, r);
+  ProfileEnd(prof, stream);
+  SCEMB_LAUNCH_CHECK();
+  return 0;
 }
 
-template <int G, int VEC, int SRC, int EPI, bool kOneHot, bool kMapped>
-void LaunchReduce(const StreamArgs& st, const RowArgs& r, bool long_range,
-                  dim3 grid, hipStream_t stream) {
-  if constexpr (LongRange(G) > G && AnyOrder<EPI>()) {
-    if (long_range) {
-      hipLaunchKernelGGL(
-          (SegReduce<G, VEC, SRC, EPI, kOneHot, kMapped, LongRange(G)>), grid,
-          dim3(kBlock), 0, stream, st, r);
-      return;
+// Whether ranges are long (LongRange), by what is known of the stream: its
+// positions `n`, the entries among them (`entries`; n if unknown) and the
+// output rows. Lookups, G against 2 * G (with SegFinish, in a graph):
+//   * runs of 4 * G entries on average cross ranges of G too often at any
+//     size: 8 and 32 columns, 50 ids per sample, 2^15 entries 13.5 and 11.0 us
+//     against 11.4 and 10.6;
+//   * shorter runs gain once there are blocks to spare: 32 and 64 columns, 20
+//     ids per sample, 2^17 entries 10.3 and 10.9 us against 10.7 and 11.9,
+//     2^19 15.7 and 18.7 against 14.2 and 17.1, 2^22 73 and 88 against 52 and
+//     75; 8 columns, 5 ids, 2^18 10.3 against 10.9, 2^20 22.2 against 18.8 (8
+//     columns and 2 ids never: 2^22 70.6 against 75.9);
+//   * a buffer that is mostly padding has half the empty blocks: 32 columns,
+//     2^18 entries in 10 * 2^18 positions, 13.5 us against 11.6.
+inline bool TakesLong(int g, int64_t entries, int64_t n, int64_t rows,
+                      bool one_hot) {
+  if (entries >= 4 * g * rows) return true;
+  if (n >= (1 << 21) && n >= 4 * entries) return true;
+  return entries >= (1 << 19) && (g >= 8 || !one_hot);
+}
+
+template <int G, int VEC, int SRC, int EPI, bool kMapped>
+int LaunchLayout(const StreamArgs& st, const RowArgs& r, int64_t entries,
+                 bool one_hot, const char* reduce_span,
+                 const char* finish_span, hipStream_t stream) {
+  constexpr int kLong = LongRange<EPI>(G);
+  if constexpr (kLong > G) {
+    if (TakesLong(G, entries, st.n, r.batch, one_hot)) {
+      return LaunchRanges<G, VEC, SRC, EPI, kMapped, kLong, false>(
+          st, r, one_hot, reduce_span, finish_span, stream);
     }
   }
-  hipLaunchKernelGGL((SegReduce<G, VEC, SRC, EPI, kOneHot, kMapped, G>), grid,
-                     dim3(kBlock), 0, stream, st, r);
+  return LaunchRanges<G, VEC, SRC, EPI, kMapped, G, (kLong > G)>(
+      st, r, one_hot, reduce_span, finish_span, stream);
 }
 
 template <int SRC, int EPI, bool kMapped>
 int LaunchSegMapped(const StreamArgs& st, RowArgs r, const SegBuffers& sb,
-                    int g, int vec, bool one_hot, const char* reduce_span,
-                    const char* finish_span, hipStream_t stream) {
+                    int64_t entries, int g, int vec, bool one_hot,
+                    const char* reduce_span, const char* finish_span,
+                    hipStream_t stream) {
   r.partials = sb.partials;
   r.block_flags = sb.flags;
   r.block_keys = sb.keys;
@@ -2559,30 +2640,11 @@ int LaunchSegMapped(const StreamArgs& st, RowArgs r, const SegBuffers& sb,
     }
     if (rc != kRtcInterpret) return rc;
   }
-  const bool long_range = AnyOrder<EPI>() && UseLongRange(g, st.n);
-  const int64_t num_blocks =
-      long_range ? CeilDiv(st.n, kBlock / g * LongRange(g)) : sb.num_blocks;
-  const dim3 grid(static_cast<uint32_t>(num_blocks));
-#define SCEMB_SEG_CASE(GG, VV)                                                \
-  if constexpr (VV == 1 || EPI != kEpiCustom)                                \
-  if (g == GG && vec == VV) {                                                \
-    int prof = ProfileBegin(reduce_span, stream);                            \
-    if (one_hot) {                                                           \
-      LaunchReduce<GG, VV, SRC, EPI, true, kMapped>(st, r, long_range, grid,  \
-                                                    stream);                  \
-    } else {                                                                 \
-      LaunchReduce<GG, VV, SRC, EPI, false, kMapped>(st, r, long_range, grid, \
-                                                     stream);                 \
-    }                                                                        \
-    ProfileEnd(prof, stream);                                                 \
-    SCEMB_LAUNCH_CHECK();                                                     \
-    if (r.single_runs) return 0;                                              \
-    prof = ProfileBegin(finish_span, stream);                                 \
-    hipLaunchKernelGGL((SegFinish<GG, VV, EPI, kMapped>), grid, dim3(kBlock), \
-                       0, stream, num_blocks, r);                             \
-    ProfileEnd(prof, stream);                                                 \
-    SCEMB_LAUNCH_CHECK();                                                     \
-    return 0;                                                                 \
+#define SCEMB_SEG_CASE(GG, VV)                                            \
+  if constexpr (VV == 1 || EPI != kEpiCustom)                            \
+  if (g == GG && vec == VV) {                                            \
+    return LaunchLayout<GG, VV, SRC, EPI, kMapped>(                       \
+        st, r, entries, one_hot, reduce_span, finish_span, stream);       \
   }
   SCEMB_SEG_CASE(4, 1) SCEMB_SEG_CASE(8, 1) SCEMB_SEG_CASE(16, 1)
   SCEMB_SEG_CASE(32, 1) SCEMB_SEG_CASE(64, 1) SCEMB_SEG_CASE(4, 4)
@@ -2748,19 +2810,20 @@ int LaunchHotReduce(const StreamArgs& st, const RowArgs& r,
   return Fail(SCEMB_ERR_INVALID_ARGUMENT, "unsupported layout");
 }
 
-// Launches SegReduce + SegFinish for the layout picked for `dim`; `one_hot`
+// Launches SegReduce + SegFinish for the layout picked for `dim`; `entries`
+// (the stream's, as far as known) selects the ranges' length, `one_hot`
 // selects the wide unroll, `mapped` the kernels that address activations
 // through the row map in `r.act` (which may hold no block at all).
 template <int SRC, int EPI>
 int LaunchSeg(const StreamArgs& st, const RowArgs& r, const SegBuffers& sb,
-              int g, int vec, bool one_hot, bool mapped,
+              int64_t entries, int g, int vec, bool one_hot, bool mapped,
               const char* reduce_span, const char* finish_span,
               hipStream_t stream) {
   if (mapped) {
-    return LaunchSegMapped<SRC, EPI, true>(st, r, sb, g, vec, one_hot,
+    return LaunchSegMapped<SRC, EPI, true>(st, r, sb, entries, g, vec, one_hot,
                                            reduce_span, finish_span, stream);
   }
-  return LaunchSegMapped<SRC, EPI, false>(st, r, sb, g, vec, one_hot,
+  return LaunchSegMapped<SRC, EPI, false>(st, r, sb, entries, g, vec, one_hot,
                                           reduce_span, finish_span, stream);
 }
 
@@ -2846,8 +2909,9 @@ int GradImpl(const GradCall& c) {
   const bool mapped = c.map != nullptr;
   if (direct) {
     if (!hb.on) {
-      return LaunchSeg<kSrcCsr, EPI>(st, r, sb, g, vec, one_hot, mapped,
-                                     "bwd_reduce", "bwd_finish", stream);
+      return LaunchSeg<kSrcCsr, EPI>(st, r, sb, entries, g, vec, one_hot,
+                                     mapped, "bwd_reduce", "bwd_finish",
+                                     stream);
     }
     rc = LaunchHotPlan(&st, hb, c.status, stream);
     if (rc != 0) return rc;
@@ -2858,13 +2922,15 @@ int GradImpl(const GradCall& c) {
     rc = ForkSide(stream, &side);
     if (rc != 0) return rc;
     const int rc_seg = LaunchSeg<kSrcCsr, EPI>(
-        st, r, sb, g, vec, one_hot, mapped, "bwd_reduce", "bwd_finish", stream);
+        st, r, sb, entries, g, vec, one_hot, mapped, "bwd_reduce",
+        "bwd_finish", stream);
     rc = LaunchHotReduce<EPI>(st, r, hb, g, vec, mapped, side);
     const int rc_join = JoinSide(stream);
     return rc != 0 ? rc : rc_seg != 0 ? rc_seg : rc_join;
   }
-  return LaunchSeg<kSrcSorted, EPI>(st, r, sb, g, vec, one_hot, mapped,
-                                    "bwd_reduce", "bwd_finish", stream);
+  return LaunchSeg<kSrcSorted, EPI>(st, r, sb, entries, g, vec, one_hot,
+                                    mapped, "bwd_reduce", "bwd_finish",
+                                    stream);
 }
 
 #endif  // __HIPCC_RTC__

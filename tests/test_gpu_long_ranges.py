@@ -1,9 +1,13 @@
-"""Lookups and updates of narrow rows at the stream length from which a
-sub-group takes a longer range of entries (segreduce.h, UseLongRange): one
-block less than that, exactly that, and a ragged last block past it, for the
-4- and 16-byte layouts, dense and per-feature activations. Tables, gradients
-and gains are small integers, for which every order of summation is exact, so
-the results equal a plain index_add bit for bit."""
+"""Lookups of narrow rows around the entries from which a sub-group takes a
+range twice as long (segreduce.h, TakesLong), for the 4-, 8- and 16-lane
+layouts with 4- and 16-byte loads, dense and per-feature activations.
+
+With tables, gradients and gains of small integers every order of summation is
+exact, and the results equal a plain index_add bit for bit (the updates of the
+same entries too; their ranges have one length). With random floats the two
+lengths still add up in one order: neither the buffer that the entries came in
+nor what the caller says of their number changes a bit, and the sums are as
+close to 64 bits as sums of short pieces are."""
 
 import numpy as np
 import pytest
@@ -24,9 +28,8 @@ from jax_tpu_embedding.sparsecore.lib.core.primitives import _device  # pylint: 
 from jax_tpu_embedding.sparsecore.lib.core.primitives import sparse_dense_matmul_csr as fwd  # pylint: disable=g-import-not-at-top,wrong-import-position
 from jax_tpu_embedding.sparsecore.lib.core.primitives import sparse_dense_matmul_grad_with_sgd as sgd  # pylint: disable=g-import-not-at-top,wrong-import-position
 
-# dim -> entries from which the range is long: 512 blocks of (lanes per row:
-# 4, 8, 16) 1024, 512, 512 entries.
-LONG = {3: 1 << 19, 16: 1 << 19, 20: 1 << 18, 13: 1 << 18, 64: 1 << 18}
+LONG = 1 << 19
+DIMS = (3, 13, 16, 20, 64)  # 4, 16, 4, 8 and 16 lanes
 
 
 def _csr(rng, n, entries, rows, batch):
@@ -55,13 +58,12 @@ def _csr(rng, n, entries, rows, batch):
 
 
 @pytest.mark.parametrize("mapped", [False, True])
-@pytest.mark.parametrize("dim", sorted(LONG))
+@pytest.mark.parametrize("dim", DIMS)
 def test_long_ranges_are_exact(dim, mapped):
   rng = np.random.default_rng(dim)
   batch, rows = 40000, 300_000 if dim < 20 else 150_000
-  for n, entries in ((LONG[dim] - 1, LONG[dim] - 9),
-                     (LONG[dim], LONG[dim] - 1000),
-                     (LONG[dim] + 777, LONG[dim] + 777)):
+  for n, entries in ((LONG - 1, LONG - 9), (LONG, LONG - 1000),
+                     (LONG + 777, LONG + 777)):
     csr, eid, sid, gains = _csr(rng, n, entries, rows, batch)
     dev = [torch.from_numpy(x).cuda() for x in csr]
     table = torch.from_numpy(rng.integers(-4, 5, size=(rows, dim))).float()
@@ -96,3 +98,45 @@ def test_long_ranges_are_exact(dim, mapped):
     sgd.tpu_sparse_dense_matmul_grad_with_sgd_primitive.bind(
         *dev, 1, t_dev, grad_dev, 0.5, **kw)
     assert torch.equal(t_dev.cpu(), table - up * 0.5)
+
+
+@pytest.mark.parametrize("dim", DIMS)
+def test_one_order_whatever_the_buffer_and_the_count(dim):
+  rng = np.random.default_rng(dim + 1)
+  batch, rows = 40000, 300_000
+  table = torch.from_numpy(
+      rng.normal(size=(rows, dim)).astype(np.float32)).cuda()
+  for entries in (LONG // 2 - 5, LONG + 4097):
+    csr, eid, sid, _ = _csr(rng, entries, entries, rows, batch)
+    gains = rng.random(entries, dtype=np.float32)
+    results = []
+    # The buffer's positions, and the entry count that the caller gives (None:
+    # unknown, the buffer's size stands in; a small count asks for the short
+    # ranges, unless the buffer is much larger).
+    for n, count in ((entries, entries), (entries, None), (entries, 1000),
+                     (3 * LONG, entries), (3 * LONG, None), (3 * LONG, 1000),
+                     (4 * LONG, 1000)):
+      dev = [torch.from_numpy(csr[0]).cuda()]
+      for x, fill in ((eid.astype(np.int32), 2**31 - 1),
+                      (sid.astype(np.int32), 2**31 - 1), (gains, np.nan)):
+        y = np.full(n, fill, x.dtype)
+        y[:entries] = x
+        dev.append(torch.from_numpy(y).cuda())
+      results.append(fwd.tpu_sparse_dense_matmul_csr_primitive.bind(
+          *dev, 1, table, device_batch_size=batch, max_ids_per_partition=n,
+          max_unique_ids_per_partition=n, num_sc_per_device=1,
+          csr_num_entries=count))
+    for k, other in enumerate(results[1:]):
+      assert torch.equal(results[0], other), (entries, k)
+    # A sum of m products: pieces of at most 16 entries (one rounding each,
+    # the products being fused), at most 16 pieces, and one addition per
+    # doubling or block after that.
+    e, s = torch.from_numpy(eid).long(), torch.from_numpy(sid).long()
+    w = torch.from_numpy(gains).double()[:, None]
+    t = table.cpu().double()
+    exact = torch.zeros(batch, dim, dtype=torch.float64)
+    size = torch.zeros(batch, dim, dtype=torch.float64)
+    exact.index_add_(0, s, t[e] * w)
+    size.index_add_(0, s, (t[e] * w).abs())
+    bound = (16 + 16 + 32) * 2.0**-24 * size
+    assert bool(((results[0].cpu().double() - exact).abs() <= bound).all())
