@@ -3349,7 +3349,10 @@ struct UniqueStack {
   int64_t view_grid = 0;
   ViewWriteArgs<K> vw;
   bool flat = false;  // one bucket, and the view holds the sort's entries
-  bool wide = false;  // flat, sorted by digits of up to kWideDigitBits
+  // Flat: sorted by digits of up to kWideDigitBits, and by work-groups of
+  // kWideBlock threads.
+  bool wide = false;
+  bool wide_block = false;
   bool small = false;  // flat, one work-group after the extraction
   FlatSmallArgs fs;
   FlatViewArgs fv;
@@ -3397,6 +3400,7 @@ int PrepareUnique(const scemb_feature_t* feats, int nf,
     const radix::DigitPlan wide =
         radix::PlanDigits(u->key_bits, radix::kWideDigitBits);
     u->wide = wide.passes < u->dp.passes;
+    u->wide_block = u->wide && M > radix::kWideSmallMax;
     if (u->wide) u->dp = wide;
   }
   // Cleared by the set-up launch: the buckets' distinct-column counts, the
@@ -3415,7 +3419,9 @@ int PrepareUnique(const scemb_feature_t* feats, int nf,
   SliceDesc* slices =
       ws.Take<SliceDesc>(static_cast<int64_t>(pl.slices.size()));
   FeatureDev* fdev = ws.Take<FeatureDev>(nf);
-  u->tiles = CeilDiv(M, u->wide ? radix::kWideTile : radix::kSortTile);
+  u->tiles = CeilDiv(M, (u->wide_block ? radix::kWideBlock
+                                       : radix::kSortBlock) *
+                            radix::kSortChunks);
   const int64_t cells = u->tiles * (int64_t{1} << u->dp.digit);
   u->hist = ws.Take<uint32_t>(cells);
   // The scans' tile sums for grouped scans; a scan too long for one is left
@@ -3613,8 +3619,8 @@ int EnqueueSmall(UniqueStack<uint32_t>* const* st, int n, hipStream_t stream) {
 
 // The stages of the stacks of one bucket (UniqueStack::flat): extraction, the
 // view, the radix passes from the view into the CSR, the distinct columns,
-// the fill plan and the padding. One extraction variant and one digit width
-// per call: digits of 9 bits where they take one pass fewer than digits of 8
+// the fill plan and the padding. One extraction variant, one work-group size
+// and one digit width per call: digits of 9 bits where they take one pass fewer than digits of 8
 // (1.7M ids, 26-bit rows: the sort's kernels 134 -> 110 us, four launches
 // fewer; 8.7M ids: 363 and 378 us, whole call 1120 and 1121 us).
 template <bool kHashed, int kBlk, int kBits>
@@ -3752,12 +3758,13 @@ template <typename K, bool kHashed>
 int EnqueueUnique(UniqueStack<K>* const* all, int num, hipStream_t stream) {
   const bool measuring = num > 0 && all[0]->measuring;
   int rc = 0;
-  std::vector<UniqueStack<K>*> rest, flat, wide, small;
+  std::vector<UniqueStack<K>*> rest, flat, wide, wide_block, small;
   for (int i = 0; i < num; ++i) {
-    (!all[i]->flat   ? rest
-     : all[i]->small ? small
-     : all[i]->wide  ? wide
-                     : flat).push_back(all[i]);
+    (!all[i]->flat        ? rest
+     : all[i]->small      ? small
+     : all[i]->wide_block ? wide_block
+     : all[i]->wide       ? wide
+                          : flat).push_back(all[i]);
   }
   if constexpr (sizeof(K) == 4) {
     if (!measuring && !small.empty()) {
@@ -3771,8 +3778,13 @@ int EnqueueUnique(UniqueStack<K>* const* all, int num, hipStream_t stream) {
       if (rc != 0) return rc;
     }
     if (!measuring && !wide.empty()) {
-      rc = EnqueueFlat<kHashed, radix::kWideBlock, radix::kWideDigitBits>(
+      rc = EnqueueFlat<kHashed, radix::kSortBlock, radix::kWideDigitBits>(
           wide.data(), static_cast<int>(wide.size()), stream);
+      if (rc != 0) return rc;
+    }
+    if (!measuring && !wide_block.empty()) {
+      rc = EnqueueFlat<kHashed, radix::kWideBlock, radix::kWideDigitBits>(
+          wide_block.data(), static_cast<int>(wide_block.size()), stream);
       if (rc != 0) return rc;
     }
   }

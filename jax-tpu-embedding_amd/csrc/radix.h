@@ -28,9 +28,15 @@ constexpr int kSortTile = kSortBlock * kSortChunks;
 constexpr int kMaxDigitBits = 8;
 // Passes of a wider digit, for key widths that then take one pass fewer: 512
 // threads and tiles of 4,096, so that a tile still holds eight elements per
-// digit on average (its writes come out bucket by bucket).
+// digit on average (its writes come out bucket by bucket). Up to kWideSmallMax
+// elements 256 threads, as in the narrow passes: such a work-group takes one
+// wave of each SIMD and half the LDS, for which a CU full of a training step's
+// reductions has room more often (1.7M ids preprocessed beside the step before:
+// 100 us for a pass, 64 with 256 threads, the loop 0.643 and 0.622 ms). Alone
+// the sizes differ little up to there (preprocessing of 1.6M ids 285 and 290
+// us; 2.4M 341 and 350, 8M 740 and 790).
 constexpr int kWideBlock = 512;
-constexpr int kWideTile = kWideBlock * kSortChunks;
+constexpr int64_t kWideSmallMax = int64_t{1} << 21;
 constexpr int kWideDigitBits = 9;
 
 template <typename K>

@@ -238,6 +238,21 @@ __host__ __device__ constexpr int Unroll() {
   return EPI == kEpiFwd ? (kOneHot ? 8 : 4)
                         : (kOneHot || EPI == kEpiSgd ? 4 : 2);
 }
+// Waves per SIMD that the reduction may take of a CU. The one-hot kernels of
+// wide rows have registers for five (88 each): four gather as fast or faster,
+// as fewer rows in flight leave more of them in the caches (26 one-hot features
+// of 128 columns, batch 65,536, lookup and Adagrad 0.520 -> 0.510 ms; Adam, 8
+// features of 131,072, 287 -> 258 us), and leave a quarter of a CU's registers
+// for kernels beside them, a training loop's preprocessing of its next batch
+// above all. That loop waits for the preprocessing when its kernels wait for
+// room (0.650 ms per step with five waves, 0.624 with four and the sort's
+// work-groups of 256 threads). Three waves gave 0.596 there, but cost an
+// Adagrad update alone up to 10%; narrower rows and updates without slots lose
+// up to 29% with four.
+template <int G, int EPI, bool kOneHot>
+__host__ __device__ constexpr int MaxWaves() {
+  return kOneHot && G >= 32 && EPI != kEpiSgd && !IsCustom<EPI>() ? 4 : 8;
+}
 // Entries per activation row up to which a batch counts as one-hot.
 constexpr int64_t kOneHotMaxEntriesPerRow = 2;
 // Streaming (nontemporal) access for data touched once per call, so the
@@ -1201,7 +1216,9 @@ __device__ __forceinline__ uint32_t FetchCold(const StreamArgs& s, bool hot,
 // one 64-bit add, the load and four fused multiply-adds.
 template <int G, int VEC, int SRC, int EPI, bool kOneHot, bool kMapped,
           int R = G>
-__global__ __launch_bounds__(kBlock) void SegReduce(StreamArgs st, RowArgs r) {
+__global__ __launch_bounds__(kBlock)
+    __attribute__((amdgpu_waves_per_eu(1, MaxWaves<G, EPI, kOneHot>())))
+    void SegReduce(StreamArgs st, RowArgs r) {
   using V = Vec<VEC>;
   using T = typename V::T;
   constexpr int P = kBlock / G;                // sub-groups
