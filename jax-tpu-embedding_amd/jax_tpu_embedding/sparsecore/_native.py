@@ -530,11 +530,19 @@ def require_gpu():
 NUM_SIDE_STREAMS = 3
 # Forking to the side streams and joining them takes about 100 us of host time
 # per call (events, waits, stream switches, marking the results), which the
-# overlap only earns back over long kernels: from this many bytes of gathered
-# and written rows on. Measured, side streams against one stream: a step that
-# gathers 6.3 GB in six widths 2.49 and 2.59 ms; 0.72 GB in two widths 636 and
-# 497 us; 0.3 GB 188 and 85 us; 20 MB 207 and 113 us.
-SIDE_STREAM_MIN_BYTES = 2_000_000_000
+# overlap only earns back over long kernels: from this many bytes of rows on,
+# an update's counted once more by half per slot variable (embedding.py).
+# Measured, one call after another, one stream and side streams. Updates in six
+# widths: 1.85 GB of rows with SGD 515 and 540 us, 1.3 GB with Adagrad (2.0
+# counted) 496 and 504, 1.85 GB (2.8) 678 and 622, 1.3 GB with Adam (2.6) 619
+# and 604, 2.9 GB with SGD 689 and 688, with Adam (5.7) 1111 and 1050; in two
+# widths: 0.5 GB 107 and 216 us, 1.1 GB with Adam (2.2) 325 and 319. Lookups
+# that group their entries first: 2.4 GB 543 and 565 us, 2.9 GB 385 and 377,
+# 3.9 GB 684 and 594. Lookups over a view lose by themselves (2.9 GB 314 and
+# 421 us, 5.8 GB 530 and 563), but not in a training step, where the host's
+# time passes beside the preprocessing (step of 6.3 GB 2.47 ms with the lookup
+# side by side, 2.52 without).
+SIDE_STREAM_MIN_BYTES = 2_500_000_000
 _side_streams = {}
 
 

@@ -771,9 +771,10 @@ def _row_bytes(spec, embedding_ids, num_entries) -> int:
   """About how many bytes of rows a stack's lookup or update moves: a row per
   CSR entry (`num_entries`, or the buffer's positions while it is not known)
   and one per sample."""
-  entries = num_entries or (embedding_ids.numel()
-                            if hasattr(embedding_ids, "numel") else
-                            np.size(embedding_ids))
+  entries = num_entries
+  if entries is None:
+    entries = (embedding_ids.numel() if hasattr(embedding_ids, "numel") else
+               np.size(embedding_ids))
   return 4 * spec.stack_embedding_dim * (entries + spec.total_sample_count)
 
 
@@ -954,11 +955,16 @@ def tpu_sparse_dense_matmul_grad(activation_gradients, preprocessed_inputs,
     return _tree.tree_unflatten(treedef, list(res))
 
   # Independent stacks of different widths update concurrently when they are
-  # large.
+  # large: table rows, and slot rows beside them, are read and written.
   counts = getattr(preprocessed_inputs, "csr_num_entries", None) or {}
+
+  def work(name):
+    slots = len(_tree.tree_leaves(embedding_variables[name])) - 1
+    rows = _row_bytes(stacked[name], eid[name], counts.get(name))
+    return rows * (2 + slots) // 2
+
   results = _native.run_per_stack(
-      stacked.keys(), update, lambda n: stacked[n].stack_embedding_dim,
-      lambda n: _row_bytes(stacked[n], eid[n], counts.get(n)))
+      stacked.keys(), update, lambda n: stacked[n].stack_embedding_dim, work)
   return {name: results[name] for name in stacked}
 
 
