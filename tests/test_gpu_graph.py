@@ -8,6 +8,8 @@ synchronisations between the replays, and compares every replay's
 activations, table and accumulator with an eager twin advanced step by step.
 """
 
+import contextlib
+
 import numpy as np
 import pytest
 
@@ -23,6 +25,7 @@ def _gpu():
   torch.cuda.set_device(0)
 
 
+from jax_tpu_embedding.sparsecore import _native  # pylint: disable=g-import-not-at-top,wrong-import-position
 from jax_tpu_embedding.sparsecore.lib.nn import embedding  # pylint: disable=g-import-not-at-top,wrong-import-position
 from jax_tpu_embedding.sparsecore.lib.nn import embedding_spec  # pylint: disable=g-import-not-at-top,wrong-import-position
 
@@ -69,10 +72,12 @@ def _workload(one_hot, seed=0, dims=(32, 32, 32), optimizer=None,
 
 @pytest.mark.parametrize("dims", [(32, 32, 32), (8, 16, 32)])
 @pytest.mark.parametrize("one_hot", [True, False])
-def test_graph_replays_equal_eager_steps(one_hot, dims):
+def test_graph_replays_equal_eager_steps(one_hot, dims, monkeypatch):
   """With stacks of three widths the lookups and updates run on forked side
-  streams (run_per_stack), so the graph also holds their fork and join."""
-  _check_graph_replays(*_workload(one_hot, dims=dims))
+  streams (run_per_stack; forced, as these are small), so the graph also holds
+  their fork and join."""
+  with _forked(monkeypatch, dims):
+    _check_graph_replays(*_workload(one_hot, dims=dims))
 
 
 def test_graph_replays_with_hot_runs(monkeypatch):
@@ -80,7 +85,6 @@ def test_graph_replays_with_hot_runs(monkeypatch):
   of hundreds of entries): its side stream's fork and join are captured
   too, and every replay equals the eager step."""
   monkeypatch.setenv("SCEMB_HOT_RUNS", "1")
-  from jax_tpu_embedding.sparsecore import _native  # pylint: disable=g-import-not-at-top
   feats, pre, init, grads = _workload(False, seed=3, vocabs=(8, 5000, 70000))
   _check_graph_replays(feats, pre, init, grads)
   # The reduction ran: one eager backward with the launch spans on (not
@@ -101,6 +105,23 @@ def test_graph_replays_with_hot_runs(monkeypatch):
     _native.profile_enable(False)
 
 
+@contextlib.contextmanager
+def _forked(monkeypatch, dims):
+  """Calls fork to side streams whatever their size, and did where there are
+  several widths, in the capture too."""
+  monkeypatch.setattr(_native, "SIDE_STREAM_MIN_BYTES", 0)
+  captured = []
+  fork = _native.side_streams
+
+  def counted(n):
+    captured.append(torch.cuda.is_current_stream_capturing())
+    return fork(n)
+
+  monkeypatch.setattr(_native, "side_streams", counted)
+  yield
+  assert (True in captured and False in captured) == (len(set(dims)) > 1)
+
+
 def _custom_adagrad(grad, table, accum, lr):
   new_accum = accum + grad * grad
   return table - lr * grad / np.sqrt(new_accum), new_accum
@@ -116,7 +137,9 @@ def test_custom_update_graph_replays_equal_eager_steps(mode, monkeypatch):
       learning_rate=0.05, custom_computation_fn=_custom_adagrad,
       slot_variable_initializers_tuple=(lambda *_: 0.1,),
       short_name_str="custom_adagrad")
-  _check_graph_replays(*_workload(False, dims=(8, 16, 32), optimizer=spec))
+  dims = (8, 16, 32)
+  with _forked(monkeypatch, dims):
+    _check_graph_replays(*_workload(False, dims=dims, optimizer=spec))
 
 
 def _check_graph_replays(feats, pre, init, grads):

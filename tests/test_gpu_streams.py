@@ -155,12 +155,17 @@ def test_preprocessing_on_a_side_stream_overlaps_steps(multi_hot):
                                     err_msg=name)
 
 
-def test_graph_replays_after_its_workspace_is_outgrown():
+@pytest.mark.parametrize("forked", [False, True])
+def test_graph_replays_after_its_workspace_is_outgrown(forked, monkeypatch):
   """A step captured on stream cs, then a larger step run eagerly on cs
   (the workspaces its calls use grow); the replays still equal an eager
-  twin. The workspaces checked are those of cs and of its side streams
-  (stacks of different widths would run there)."""
-  small, large = _specs(512), _specs(32768, dim=128)
+  twin. The workspaces checked are those of cs or, for stacks of different
+  widths forked to side streams (forced, as these are small), of those."""
+  if forked:
+    monkeypatch.setattr(_native, "SIDE_STREAM_MIN_BYTES", 0)
+    small, large = _specs_three_stacks(512), _specs_three_stacks(32768, 8)
+  else:
+    small, large = _specs(512), _specs(32768, dim=128)
   rng = np.random.default_rng(21)
   pre_s, _ = embedding.preprocess_sparse_dense_matmul_input(
       _ids(rng, small, True), None, small, 1, 1, num_sc_per_device=1)
@@ -181,7 +186,8 @@ def test_graph_replays_after_its_workspace_is_outgrown():
   torch.cuda.synchronize()
   dev = torch.cuda.current_device()
   sides = _native._side_streams.get((dev, cs.cuda_stream), [])  # pylint: disable=protected-access
-  keys = [(dev, s.cuda_stream) for s in [cs] + list(sides)]
+  assert bool(sides) or not forked
+  keys = [(dev, s.cuda_stream) for s in (sides if forked else [cs])]
   bufs = _native.WORKSPACE._buf  # pylint: disable=protected-access
   captured = {k: bufs[k] for k in keys if k in bufs}
   assert captured
@@ -203,10 +209,10 @@ def test_graph_replays_after_its_workspace_is_outgrown():
     _assert_same(eager, graphed, f"replay {i}")
 
 
-def _specs_three_stacks(batch):
+def _specs_three_stacks(batch, scale=1):
   """Three tables of different dims: three stacks in one call."""
   tables = [embedding_spec.TableSpec(
-      name=f"d{dim}", vocabulary_size=v, embedding_dim=dim,
+      name=f"d{dim}", vocabulary_size=v, embedding_dim=dim * scale,
       initializer=embedding_spec.zeros,
       optimizer=embedding_spec.AdagradOptimizerSpec(0.05), combiner="sum",
       max_ids_per_partition=1 << 20, max_unique_ids_per_partition=1 << 20)
@@ -221,7 +227,8 @@ def _specs_three_stacks(batch):
 @pytest.mark.parametrize("multi_hot", [False, True])
 def test_stacks_on_side_streams_equal_one_stream(multi_hot, monkeypatch):
   """The stacks of one call are enqueued on forked side streams (the
-  preprocessing, the lookups and the updates); the CSR (compared region),
+  preprocessing, the lookups and the updates; forced, as these are small); the
+  CSR (compared region),
   the stats and a training step equal those of the same calls with every
   stack on the calling stream."""
   feats = _specs_three_stacks(4096)
@@ -229,14 +236,21 @@ def test_stacks_on_side_streams_equal_one_stream(multi_hot, monkeypatch):
   ids = _ids(np.random.default_rng(21), feats, multi_hot)
   grads = _grads(feats, 6)
   init = _state(feats, 4)
+  monkeypatch.setattr(_native, "SIDE_STREAM_MIN_BYTES", 0)
+  forks = []
+  fork = _native.side_streams
+  monkeypatch.setattr(_native, "side_streams",
+                      lambda n: forks.append(n) or fork(n))
   runs = []
   for sides in (_native.NUM_SIDE_STREAMS, 0):
     monkeypatch.setattr(_native, "NUM_SIDE_STREAMS", sides)
+    forks.clear()
     pre, stats = embedding.preprocess_sparse_dense_matmul_input(
         ids, None, feats, 1, 1, num_sc_per_device=1)
     state = _clone(init)
     acts = _step(pre, state, feats, grads)
     torch.cuda.synchronize()
+    assert any(n > 0 for n in forks) == (sides > 0)
     runs.append((_csr(pre), stats, state,
                  [a.cpu().numpy() for a in acts]))
   (csr_a, stats_a, state_a, acts_a), (csr_b, stats_b, state_b, acts_b) = runs
