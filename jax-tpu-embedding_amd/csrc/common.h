@@ -104,28 +104,22 @@ __device__ __forceinline__ uint64_t LaneMaskLt() {
   return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
-// The lanes of `among` whose v equals this lane's in its low `bits` bits (the
-// compile-time kBits, if set: unrolled). One ballot per bit; this form takes
-// four vector instructions per bit (bit-field extract, compare, and one
-// three-operand logic instruction per half of the mask), where selecting the
-// ballot or its complement as a 64-bit value took nine.
-template <int kBits = 0>
-__device__ __forceinline__ uint64_t MatchLanes(uint64_t among, uint32_t v,
-                                               int bits) {
+// The lanes of `among` whose v equals this lane's in its low kBits bits. One
+// ballot per bit; this form takes four vector instructions per bit (bit-field
+// extract, compare, and one three-operand logic instruction per half of the
+// mask), where selecting the ballot or its complement as a 64-bit value took
+// nine.
+template <int kBits>
+__device__ __forceinline__ uint64_t MatchLanes(uint64_t among, uint32_t v) {
   uint32_t lo = static_cast<uint32_t>(among);
   uint32_t hi = static_cast<uint32_t>(among >> 32);
-  const auto step = [&](int b) {
+#pragma unroll
+  for (int b = 0; b < kBits; ++b) {
     const uint32_t t = static_cast<uint32_t>(
         __builtin_amdgcn_sbfe(static_cast<int>(v), b, 1));
     const uint64_t ones = __ballot(t != 0);
     lo &= ~(static_cast<uint32_t>(ones) ^ t);
     hi &= ~(static_cast<uint32_t>(ones >> 32) ^ t);
-  };
-  if constexpr (kBits > 0) {
-#pragma unroll
-    for (int b = 0; b < kBits; ++b) step(b);
-  } else {
-    for (int b = 0; b < bits; ++b) step(b);
   }
   return (static_cast<uint64_t>(hi) << 32) | lo;
 }
@@ -191,7 +185,9 @@ __global__ __launch_bounds__(A::kBlock) void GroupedKernel(Group<A> g) {
   A::Run(g.a[p], blockIdx.x - g.first[p], g.first[p + 1] - g.first[p]);
 }
 
-// One problem alone, whose arguments are an eighth as long.
+// One problem alone, whose arguments are an eighth as long (a training loop
+// that preprocesses 1.7M ids beside each step, 20 such launches: 0.656 -> 0.650
+// ms).
 template <typename A>
 __global__ __launch_bounds__(A::kBlock) void SingleKernel(A a) {
   A::Run(a, blockIdx.x, gridDim.x);

@@ -2465,7 +2465,7 @@ struct FlatSmallArgs {
         const bool active = w0 + c * kWave + lane < w1;
         const uint32_t v = (key[c] >> shift) & mask;
         const uint64_t match =
-            MatchLanes<kSmallBits>(__ballot(active), v, 0);
+            MatchLanes<kSmallBits>(__ballot(active), v);
         const bool leader = active && (match & lt) == 0;
         uint32_t before = 0;
         if (leader) {

@@ -244,7 +244,7 @@ __device__ __forceinline__ void RadixScatterBody(
     const bool active = act[c];
     const uint32_t d = active ? Digit(key[c], shift, mask) : 0u;
     // A narrower digit's upper bits are zero.
-    const uint64_t match = MatchLanes<kBits>(__ballot(active), d, 0);
+    const uint64_t match = MatchLanes<kBits>(__ballot(active), d);
     // The lowest lane of each digit group bumps the wave's counter; the
     // group reads the count before the bump from it.
     const bool leader = active && (match & lt) == 0;
@@ -408,7 +408,7 @@ __device__ __forceinline__ void BucketLdsPass(
     const bool active = w0 + c * kWave + lane < w1;
     const uint32_t v = (static_cast<uint32_t>(key[c]) >> shift) & mask;
     const uint64_t match =
-        MatchLanes<kBucketDigitMax>(__ballot(active), v, 0);
+        MatchLanes<kBucketDigitMax>(__ballot(active), v);
     const bool leader = active && (match & lt) == 0;
     uint32_t before = 0;
     if (leader) {

@@ -20,7 +20,8 @@
 // SegReduce gives every 256-thread block a fixed slice of the stream (perfect
 // load balance however skewed the keys are). A block is split into
 // P = 256 / G sub-groups of G lanes; sub-group s owns entries [s*R, s*R + R)
-// of the slice and its lanes cover G * VEC columns of a row (16-byte loads).
+// of the slice (R is G, or in lookups also 2 * G) and its lanes cover G * VEC
+// columns of a row (16-byte loads).
 // A sub-group walks its entries a few at a time, issuing all row loads of a
 // batch (and, for runs that end inside the batch, the table / accumulator
 // loads of the update) before accumulating. A run that is complete inside
